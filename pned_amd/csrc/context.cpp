@@ -906,11 +906,6 @@ int check_same_layout(const pned_vec *x, const pned_vec *y)
     return PNED_OK;
 }
 
-bool default_large(const pned_ctx *ctx, int colbits)
-{
-    return (double)ctx->dim * (double)(1ull << colbits) > (double)(1ull << 25);
-}
-
 // The lane program of a diagonal (see DiagDev): groups sorted by weight class, so the
 // kernel sums a class's popcounts as integers and converts them once.
 static void build_diag_program(DiagDev &dh)
@@ -1003,13 +998,17 @@ int ensure_s12_plan(pned_ctx *ctx, int colbits, int dtype)
     if (ctx->plan_colbits == colbits && ctx->plan_dtype == dtype) return PNED_OK;
     ctx->plan_req_colbits = -1;   // set again by ensure_s12_plan_cols once it has chosen
     // the whole tile sits in LDS (160 KB on gfx950): 2^13 complex128 or 2^14 complex64.
-    // Untuned default (the autotuner's usual choice): vectors of up to 2^25 elements two
-    // bits below that limit (small tiles, 256 threads, more blocks in flight), larger
-    // vectors one bit below (1024 threads)
+    // Untuned default: complex128 2^11-state tiles up to 2^21 elements (enough tiles to fill
+    // the compute units), 2^12 above; complex64 2^12 up to 2^25 elements, 2^13 above (its rounded
+    // sums follow the passes, so the tiles are part of its results); each one bit more where
+    // that saves a pass
     const int kmax = (dtype == PNED_C128) ? 13 : 14;
     int K = ctx->tune_tile_bits;
     const bool untuned = K <= 0;
-    if (untuned) K = default_large(ctx, colbits) ? kmax - 1 : kmax - 2;
+    if (untuned) {
+        const double elems = (double)ctx->dim * (double)(1ull << colbits);
+        K = elems > (double)(1ull << (dtype == PNED_C128 ? 21 : 25)) ? kmax - 1 : kmax - 2;
+    }
     if (K > kmax) K = kmax;
     int L = ctx->tune_low_bits > 0 ? ctx->tune_low_bits : 3;
     PNED_TRY(s12_make_passes(ctx->s12, colbits, K, L));

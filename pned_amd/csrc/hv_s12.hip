@@ -46,7 +46,9 @@ struct PassArgs {
     //      partials [|w - alpha s v1|^2, 0]
     int lz_mode;
     const double *lz_prd;
+    int nt;                // term-major kernel: NT_V1 / NT_V0 streams
 };
+constexpr int NT_V1 = 1, NT_V0 = 2;
 
 // Per-pass address tables in device memory (read with scalar loads):
 //   lo[t]  memory-index offset of thread t's slot (tile bits 0..LT-1)
@@ -63,6 +65,27 @@ struct PassDev {
 template <typename R> struct C2;
 template <> struct C2<double> { using T = double2; };
 template <> struct C2<float> { using T = float2; };
+
+// vector elements with a non-temporal hint (streams that the caches should not keep)
+template <typename V>
+__device__ __forceinline__ V ld_nt(const V *p)
+{
+    using X = decltype(V::x) __attribute__((ext_vector_type(2)));
+    const X t = __builtin_nontemporal_load(reinterpret_cast<const X *>(p));
+    V v;
+    v.x = t.x;
+    v.y = t.y;
+    return v;
+}
+template <typename V>
+__device__ __forceinline__ void st_nt(V *p, const V &v)
+{
+    using X = decltype(V::x) __attribute__((ext_vector_type(2)));
+    X t;
+    t.x = v.x;
+    t.y = v.y;
+    __builtin_nontemporal_store(t, reinterpret_cast<X *>(p));
+}
 
 __device__ __forceinline__ double diag_value_re(const DiagDev &d, uint32_t s, double &im)
 {
@@ -319,8 +342,20 @@ __global__ __launch_bounds__(TPB) void hv_s12_pass(const typename C2<Real>::T *_
 // and S v0 values are live next to the R prefetched v1 values of the next tile; a sweep's
 // v0 values are in flight while its terms are applied.  Accumulates in Real (FP64 for complex128, FP32 for complex64
 // storage); the <x|Hx> partials are FP64.
+//
+// Non-temporal streams (nt): where the two vectors together exceed the 256 MB Infinity Cache, v0
+// is read and written with the non-temporal hint, and v1 as well where it alone exceeds it, so
+// a v1 that fits is still there when the next pass reads it (N=24 with field, complex128: 605 ->
+// 565 us at 1024 threads; N=28 9.40 -> 9.08 ms, N=30 45.4 -> 45.0 ms; complex64 runs of 64 bytes
+// lose, 5.80 -> 6.48 ms at N=28, because a line's other half is fetched again).
+//
+// 2^12-state complex128 tiles on 512 threads are held to 128 VGPRs (sweeps of 4 slots): two
+// blocks then share a CU (64 KB of LDS each) and one's loads run under the other's barriers
+// (N=24 with field: 677 -> 533 us per H.v; one 1024-thread block per CU 565 us).
+template <typename Real, int TPB, int R>
+constexpr int TM_WAVES = (sizeof(Real) == 8 && TPB == 512 && R == 8) ? 4 : 1;
 template <typename Real, int TPB, int R, int S>
-__global__ __launch_bounds__(TPB) void hv_s12_tm(const typename C2<Real>::T *__restrict__ v1,
+__global__ __launch_bounds__(TPB, (TM_WAVES<Real, TPB, R>)) void hv_s12_tm(const typename C2<Real>::T *__restrict__ v1,
                                                  typename C2<Real>::T *__restrict__ v0,
                                                  const TmTerm *__restrict__ terms,
                                                  const DiagDev *__restrict__ diagp,
@@ -369,19 +404,34 @@ __global__ __launch_bounds__(TPB) void hv_s12_tm(const typename C2<Real>::T *__r
 
     double pr_re = 0.0, pr_im = 0.0;
     Real xr[R], xi[R];
+    const bool nt1 = a.nt & NT_V1, nt0 = a.nt & NT_V0;
     auto fetch_x = [&](uint64_t b) {
-        static_for<R>([&](auto I) {
-            const V t = v1[b | pd->hi[I]];
-            xr[I] = t.x;
-            xi[I] = t.y;
-        });
+        if (nt1)
+            static_for<R>([&](auto I) {
+                const V t = ld_nt(&v1[b | pd->hi[I]]);
+                xr[I] = t.x;
+                xi[I] = t.y;
+            });
+        else
+            static_for<R>([&](auto I) {
+                const V t = v1[b | pd->hi[I]];
+                xr[I] = t.x;
+                xi[I] = t.y;
+            });
     };
     auto fetch_y = [&](uint64_t b, int r0, Real *yr, Real *yi) {
-        static_for<S>([&](auto I) {
-            const V t = v0[b | pd->hi[r0 + I]];
-            yr[I] = t.x;
-            yi[I] = t.y;
-        });
+        if (nt0)
+            static_for<S>([&](auto I) {
+                const V t = ld_nt(&v0[b | pd->hi[r0 + I]]);
+                yr[I] = t.x;
+                yi[I] = t.y;
+            });
+        else
+            static_for<S>([&](auto I) {
+                const V t = v0[b | pd->hi[r0 + I]];
+                yr[I] = t.x;
+                yi[I] = t.y;
+            });
     };
     // each block takes a contiguous range of tiles: consecutive tiles of a block differ in the
     // lowest outer bits, so its runs follow each other in memory (measured at N=32: a few per
@@ -587,6 +637,7 @@ __global__ __launch_bounds__(TPB) void hv_s12_tm(const typename C2<Real>::T *__r
                     ai[I] *= colsc;
                 });
             }
+            // ar, ai become the values to store (nothing is stored in lz_mode 1)
             static_for<S>([&](auto I) {
                 const V x = tile[tid + TPB * (r0 + I)];
                 if (a.lz_mode == 2) {
@@ -596,27 +647,30 @@ __global__ __launch_bounds__(TPB) void hv_s12_tm(const typename C2<Real>::T *__r
                     const double wr = wr0 - (lar * xr_ - lai * xi_);
                     const double wi = wi0 - (lar * xi_ + lai * xr_);
                     pr_re = fma(wr, wr, fma(wi, wi, pr_re));
-                    V o;
-                    o.x = (Real)(wr0 - lar * xr_);
-                    o.y = (Real)(wi0 - lar * xi_);
-                    v0[tb0 | pd->hi[r0 + I]] = o;
+                    ar[I] = (A)(wr0 - lar * xr_);
+                    ai[I] = (A)(wi0 - lar * xi_);
                 } else {
                     const double hr = (double)ar[I], hi = (double)ai[I];
                     pr_re += (double)x.x * hr + (double)x.y * hi;
                     pr_im += (double)x.x * hi - (double)x.y * hr;
-                    if (a.lz_mode != 1) {
-                        V o;
-                        if (rd0) {
-                            o.x = (Real)fma(ys, (A)ycr[I], ar[I]);
-                            o.y = (Real)fma(ys, (A)yci[I], ai[I]);
-                        } else {
-                            o.x = (Real)ar[I];
-                            o.y = (Real)ai[I];
-                        }
-                        v0[tb0 | pd->hi[r0 + I]] = o;
+                    if (rd0) {
+                        ar[I] = fma(ys, (A)ycr[I], ar[I]);
+                        ai[I] = fma(ys, (A)yci[I], ai[I]);
                     }
                 }
             });
+            auto value = [&](auto I) {
+                V o;
+                o.x = (Real)ar[I];
+                o.y = (Real)ai[I];
+                return o;
+            };
+            if (a.lz_mode != 1) {
+                if (nt0)
+                    static_for<S>([&](auto I) { st_nt(&v0[tb0 | pd->hi[r0 + I]], value(I)); });
+                else
+                    static_for<S>([&](auto I) { v0[tb0 | pd->hi[r0 + I]] = value(I); });
+            }
         });
         __syncthreads();
     }
@@ -739,7 +793,7 @@ static int dispatch_tm(pned_ctx *ctx, int TPB, int R, const void *v1, void *v0, 
     if (TPB == T_ && R == R_) return launch_tm<Real, T_, R_, S_>(ctx, v1, v0, tm, ddiag, pd, a, partial, grid);
     if constexpr (sizeof(Real) == 8) {
         PNED_CASE(256, 16, 8) PNED_CASE(256, 8, 8) PNED_CASE(256, 4, 4) PNED_CASE(256, 2, 2) PNED_CASE(256, 1, 1)
-        PNED_CASE(512, 16, 8) PNED_CASE(512, 8, 8) PNED_CASE(512, 4, 4) PNED_CASE(512, 2, 2) PNED_CASE(512, 1, 1)
+        PNED_CASE(512, 16, 8) PNED_CASE(512, 8, 4) PNED_CASE(512, 4, 4) PNED_CASE(512, 2, 2) PNED_CASE(512, 1, 1)
         PNED_CASE(1024, 8, 4) PNED_CASE(1024, 4, 4) PNED_CASE(1024, 2, 2) PNED_CASE(1024, 1, 1)
     } else {
         PNED_CASE(256, 32, 16) PNED_CASE(256, 16, 16) PNED_CASE(256, 8, 8) PNED_CASE(256, 4, 4)
@@ -756,12 +810,16 @@ static int dispatch_tm(pned_ctx *ctx, int TPB, int R, const void *v1, void *v0, 
 // Tile-coordinate term table of one pass (see TmTerm), sorted into the term-major
 // kernel's categories: 0 real, 1 real with register selector bits, 2 complex, 3 complex
 // with register selector bits (batch contexts: every term complex).  ncat gets the counts.
+// The order in which a state sums its terms is a function of the plan and of order_tpb alone,
+// whatever the thread count: the categories sort by the register bits that order_tpb threads
+// would leave (the looser loop of 1 and 3 is right for every selector; where TPB leaves more
+// register bits than order_tpb, all real or complex terms take it).
 // colbits: the plan's column bits; outer selector bits at or above them sit gap bits higher
 // in memory (column groups)
-static void build_tm_terms(const S12Plan &pl, const PassPlan &pp, int TPB, int colbits, int gap,
+static void build_tm_terms(const S12Plan &pl, const PassPlan &pp, int TPB, int order_tpb, int colbits, int gap,
                            std::vector<TmTerm> &out, int ncat[4])
 {
-    const int LT = __builtin_ctz(TPB);
+    const int LT = __builtin_ctz(TPB), LO = __builtin_ctz(order_tpb);
     uint64_t tilemask = 0;
     for (int b : pp.tb) tilemask |= 1ull << b;
     std::vector<TmTerm> cat[4];
@@ -785,12 +843,19 @@ static void build_tm_terms(const S12Plan &pl, const PassPlan &pp, int TPB, int c
         t.c0i = d.c0i;
         t.c1r = d.c1r;
         t.c1i = d.c1i;
-        cat[(cx ? 2 : 0) + (t.shi != 0 ? 1 : 0)].push_back(t);
+        cat[(cx ? 2 : 0) + ((stile >> LO) != 0 ? 1 : 0)].push_back(t);
     }
     for (int c = 0; c < 4; ++c) {
         ncat[c] = (int)cat[c].size();
         out.insert(out.end(), cat[c].begin(), cat[c].end());
     }
+    for (int c = 0; c < 4; c += 2)
+        for (const TmTerm &t : cat[c])
+            if (t.shi != 0) {
+                ncat[c + 1] += ncat[c];
+                ncat[c] = 0;
+                break;
+            }
 }
 
 // ------------------------------------------------------------------------------------
@@ -828,6 +893,41 @@ static double *noalloc_scratch(int device)
     if (device < 0 || device >= NOALLOC_MAX_DEVICES) return nullptr;
     std::lock_guard<std::mutex> lock(g_scratch_mu);
     return g_scratch_ptr[device];
+}
+
+// Infinity Cache, shared by the XCDs
+constexpr size_t CACHE_BYTES = (size_t)256 << 20;
+
+// consecutive low bits of an ascending bit list: runs of 2^n elements are contiguous
+static int contiguous_bits(const std::vector<int> &b)
+{
+    int n = 0;
+    while (n < (int)b.size() && b[n] == n) ++n;
+    return n;
+}
+
+// Threads of the untuned term-major plan, by its tile size (complex128 figures: one column with
+// field, us per H.v).  Up to 2^18 elements 256 threads: other counts sum <v1|H v1> in another
+// order, and a Lanczos run over such short vectors amplifies the last bit (2^16 states, 40 steps:
+// to 1e-7).  2^12-state tiles 1024 threads up to 2^21 elements (N=20 57.9, on 512 68), 512 above
+// (N=24 533 against 565: two blocks per CU), but 1024 in batches (N=20 with 8 columns 277 against
+// 344).  2^13 1024 (N=28 9.08 ms, on 512 13.9).  complex64: 2^12 512 (N=24 383, on 1024 472), 2^13
+// 1024 (N=28 5.8 ms), 2^14 512 (1024 spill; N=24 with 64 columns 28.7 against 31.7 ms).
+static int default_threads(const pned_ctx *ctx, const S12Plan &pl, int colbits, bool c128)
+{
+    const int K = pl.passes.empty() ? 12 : pl.passes[0].K;
+    const double elems = (double)ctx->dim * (double)(1ull << colbits);
+    // one tile in all: its block is all there is to sum (2^12 states: 46 us on 256, 34 on 1024)
+    if (K <= 11 || (elems <= (double)(1ull << 18) && K < ctx->n + colbits)) return 256;
+    if (!c128) return K == 13 ? 1024 : 512;
+    if (K == 12 && elems > (double)(1ull << 21) && colbits == 0) return 512;
+    return 1024;
+}
+
+// the thread count whose register slots order a pass's terms (see build_tm_terms)
+static int order_threads(const pned_ctx *ctx, int colbits)
+{
+    return (double)ctx->dim * (double)(1ull << colbits) > (double)(1ull << 25) ? 1024 : 256;
 }
 
 // noalloc: the caller's plan, pass tables and buffers must already exist; partials go to
@@ -892,11 +992,12 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
         PNED_TRY(ensure_result(ctx, 4 * (size_t)nvec + 8));
     }
     double *const part_base = noalloc ? part_ext : ctx->d_partial;
+    const bool c128 = v1->dtype == PNED_C128;
+    const size_t esz = c128 ? 16 : 8;
     // per-pass address tables (rebuilt when the plan or the thread count changes)
     const int TPBpref = (ctx->tune_threads == 256 || ctx->tune_threads == 512 || ctx->tune_threads == 1024)
                             ? ctx->tune_threads
-                            : (ctx->s12_kernel == 1 && default_large(ctx, colbits) ? 1024
-                                                                                    : (ctx->s12_kernel == 1 ? 256 : 512));
+                            : (ctx->s12_kernel == 1 ? default_threads(ctx, pl, colbits, c128) : 512);
     std::vector<int> tpb(npass), rr(npass);
     for (int p = 0; p < npass; ++p) {
         int T = TPBpref;
@@ -944,8 +1045,11 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
         }
         std::vector<TmTerm> tmh;
         ctx->tm_ncat.assign(4 * (size_t)npass, 0);
-        for (int p = 0; p < npass; ++p)
-            build_tm_terms(pl, pl.passes[p], tpb[p], cg, gap, tmh, &ctx->tm_ncat[4 * p]);
+        for (int p = 0; p < npass; ++p) {
+            int T = ctx->tune_threads > 0 ? TPBpref : order_threads(ctx, colbits);
+            while (T > 16 && T > (1 << pl.passes[p].K)) T >>= 1;
+            build_tm_terms(pl, pl.passes[p], tpb[p], T, cg, gap, tmh, &ctx->tm_ncat[4 * p]);
+        }
         if (tmh.empty()) tmh.push_back(TmTerm{});
         PNED_HIP(hipStreamSynchronize(ctx->stream));
         if (ctx->pd_dev) PNED_HIP(hipFree(ctx->pd_dev));
@@ -974,19 +1078,24 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
         ctx->pd_gap = gap;
     }
     // blocks per pass: at least 8 contiguous tiles each (so a block's next-tile loads overlap
-    // its terms for most of its tiles) while that leaves 256 or more, at most grid_cap.  At
-    // N=24 (2048 tiles of 2^13) 256 blocks ran 0.524 ms per H.v against 0.532 with 1024 and
-    // 0.554 with 2048; at N=32 4096 blocks of 128 tiles beat 1024 and 256 by about 0.5 ms
+    // its terms for most of its tiles) while that leaves one block per CU or more (two where
+    // two fit a CU), at most grid_cap.  At N=24 (2048 tiles of 2^13) 256 blocks ran 0.524 ms per
+    // H.v against 0.532 with 1024 and 0.554 with 2048; at N=32 4096 blocks of 128 tiles beat 1024
+    // and 256 by about 0.5 ms
     auto pass_grid = [&](int p) {
         const uint64_t tc = 1ull << pl.passes[p].ob.size();
-        const uint64_t want = std::max<uint64_t>(256, tc / 8);
+        const uint64_t fill = (tpb[p] <= 512 && esz << pl.passes[p].K <= LDS_LIMIT / 2) ? 512 : 256;
+        const uint64_t want = std::max<uint64_t>(fill, tc / 8);
         return (int)std::min<uint64_t>(std::min<uint64_t>(tc, want), (uint64_t)grid_cap);
     };
     // partial rows: per column group [pass][block] of 2 ncol_t values, the groups one after another
     int rows_grp = 0;
     for (int p = 0; p < npass; ++p) rows_grp += pass_grid(p);
-    const bool c128 = v1->dtype == PNED_C128;
-    const size_t esz = c128 ? 16 : 8;
+    // the non-temporal streams (see hv_s12_tm): whole 128-byte lines only
+    const size_t vec_bytes = esz * (size_t)ctx->dim * (size_t)nvec;
+    const int lowrun = pl.passes.empty() ? 0 : contiguous_bits(pl.passes[0].tb);
+    int nt = 0;
+    if (2 * vec_bytes > CACHE_BYTES && (esz << lowrun) >= 128) nt = vec_bytes > CACHE_BYTES ? NT_V1 | NT_V0 : NT_V0;
     int total_rows = 0;
     for (int p = 0; p < npass; ++p) {
         const PassPlan &pp = pl.passes[p];
@@ -1009,6 +1118,7 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
         a.yscale = d_yscale;
         for (int c = 0; c < 4; ++c) a.ncat[c] = ctx->tm_ncat[4 * p + c];
         a.ngroups = ctx->diag_host.ngroups;
+        a.nt = nt;
         const int TPB = tpb[p], R = rr[p];
         const int grid = pass_grid(p);
         const PassDev *pdp = reinterpret_cast<const PassDev *>(ctx->pd_dev) + p;

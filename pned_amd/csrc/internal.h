@@ -59,7 +59,7 @@ struct DevTerm {
 // A term as the term-major pass kernel reads it, in the coordinates of one pass's tile
 // (tile slot j = thread + TPB * register): the flip mask and the selector split into
 // thread bits (lo), register bits (hi) and, for the selector, outer memory bits.
-struct TmTerm {
+struct alignas(64) TmTerm {   // one scalar-cache line
     uint32_t mlo, mhi;   // flip mask: thread bits, register bits (>> log2 TPB)
     uint32_t slo, shi;   // selector mask: thread bits, register bits
     uint64_t sout;       // selector mask on the outer memory-index bits
@@ -332,8 +332,6 @@ int intalv_xy_apply(pned_ctx *ctx, const pned_vec *x, pned_vec *v, const double 
 // intalv_xy over the full q^N space: v = sum_j e^{i q.r_j} S^{ipm}_j x (ladder factors)
 int intalv_pm_apply(pned_ctx *ctx, const pned_vec *x, pned_vec *v, const double *qv, const double *site_vec, int ipm);
 int refresh_sector_terms(pned_ctx *ctx);   // after the bond matrices change
-// untuned tile defaults: true for vectors above 2^25 elements (dim x columns)
-bool default_large(const pned_ctx *ctx, int colbits);
 int upload_batch_coefficients(pned_ctx *ctx);
 // sums the rows of ctx->d_partial [nrows][ncol2] into ctx->d_result[0..ncol2): 256 threads
 // per column, fixed strides and a fixed tree (the same partials give the same sums)

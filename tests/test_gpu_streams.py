@@ -1,0 +1,32 @@
+"""Untuned S=1/2 plans above the cached sizes (tile size, threads and non-temporal streams by
+vector size) against the state-major kernel on the same vectors."""
+import numpy as np
+import pytest
+
+from pned_amd import gpu, lattice, model
+
+pytestmark = pytest.mark.gpu
+
+
+# 2^22 elements: first size with 2^12-state tiles; 256 MiB (16 columns): v0 non-temporal, v1
+# cached; 1 GiB and 512 MiB: both non-temporal where the runs are whole lines (complex64 with
+# one column reads 64-byte runs)
+@pytest.mark.parametrize("spec,cols,dtype", [("1x11", 1, gpu.C128), ("2x5", 16, gpu.C128), ("1x13", 1, gpu.C128),
+                                             ("1x13", 1, gpu.C64), ("2x5", 64, gpu.C64)])
+def test_untuned_plan_matches_state_major(spec, cols, dtype):
+    cl = lattice.get_cluster(spec)
+    ctx = gpu.Context(model.build_operator(cl, 20, 126.0, field=0.1))
+    x, a, b = (ctx.vector(cols, dtype) for _ in range(3))
+    ctx.set_initial_vec(x, 5)
+    ctx.set_initial_vec(a, 6)
+    b.copy_from(a)
+    pa = np.atleast_1d(ctx.p_mltply_v3(x, a, 0.03))
+    ctx.s12_kernel(0)
+    pb = np.atleast_1d(ctx.p_mltply_v3(x, b, 0.03))
+    # about 80 terms a state, each kernel rounding once a term in the storage precision
+    tol = 1e-13 if dtype == gpu.C128 else 2e-6
+    nb = np.sqrt(np.atleast_1d(ctx.calc_vec_inprdct(b, b)).real)
+    ctx.axpby(np.full(cols, -1.0 + 0j), b, np.full(cols, 1.0 + 0j), a)
+    nd = np.sqrt(np.atleast_1d(ctx.calc_vec_inprdct(a, a)).real)
+    assert np.all(nd <= tol * nb), (nd, nb)
+    assert np.all(np.abs(pa - pb) <= tol * nb)   # |<x|Hx>| <= |Hx| for the unit x
