@@ -39,52 +39,98 @@ __device__ __forceinline__ double sector_diag(const DiagDev &d, uint32_t s, doub
     return re;
 }
 
-__global__ __launch_bounds__(256) void hv_sector_kernel(const double2 *__restrict__ v1, double2 *__restrict__ v0,
+// One thread per output index.  Bound by the vector-memory address path: a partner costs one
+// 16-byte gather (16 cycles a wave) beside its arithmetic, so the two half tables sit in LDS
+// (rank as 16 bits) and not in three dependent global reads a partner, and SEC_U partners are in
+// flight at a time.  v0 = y v0 + H (x v1) with the optional device factors xs, ys.  REAL: no
+// coefficient and no diagonal weight has an imaginary part (their products are left out).
+// N=24 at k=12 (2704156 states, Heisenberg), us a call: 154 -> 108; N=28 at k=14 2632 -> 1740.
+constexpr int SEC_U = 4;
+template <bool REAL, bool LDS, int TPB>
+__global__ __launch_bounds__(TPB) void hv_sector_kernel(const double2 *__restrict__ v1, double2 *__restrict__ v0,
                                                         const uint32_t *__restrict__ list1,
                                                         const uint32_t *__restrict__ rank,
                                                         const uint32_t *__restrict__ offset,
                                                         const SectorTerm *__restrict__ terms, int nterm,
-                                                        const DiagDev *__restrict__ diagp, int ihf, double shift,
-                                                        int fresh, uint64_t dim, double *__restrict__ partial)
+                                                        const DiagDev *__restrict__ diagp, int ihf, int ihf0,
+                                                        double shift, int fresh, uint64_t dim,
+                                                        const double *__restrict__ xs, const double *__restrict__ ys,
+                                                        double *__restrict__ partial)
 {
-    __shared__ double red[512];
+    extern __shared__ uint32_t sec_smem[];
+    __shared__ double red[2 * TPB];
+    const int tid = threadIdx.x;
     const uint32_t right = (1u << ihf) - 1u;
+    uint32_t *off = sec_smem;
+    uint16_t *rk = reinterpret_cast<uint16_t *>(sec_smem + (LDS ? (1u << ihf0) : 0u));
+    if (LDS) {
+        for (uint32_t i = tid; i < (1u << ihf0); i += TPB) off[i] = offset[i];
+        for (uint32_t i = tid; i <= right; i += TPB) rk[i] = (uint16_t)rank[i];
+        __syncthreads();
+    }
     const DiagDev &dg = *diagp;
+    const double x_s = xs ? *xs : 1.0, y_s = ys ? *ys : 1.0;
     double pr_re = 0.0, pr_im = 0.0;
-    const uint64_t stride = (uint64_t)blockDim.x * gridDim.x;
-    for (uint64_t l = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; l < dim; l += stride) {
-        const uint32_t s = list1[l];
-        const double2 x = v1[l];
-        double di;
-        const double dr = sector_diag(dg, s, di) + shift;
-        double ar = dr * x.x - di * x.y, ai = dr * x.y + di * x.x;
-        for (int t = 0; t < nterm; ++t) {
-            const SectorTerm T = terms[t];
-            if (__popc(s & T.mask) != 1) continue;   // partner outside the sector: coefficient 0
-            const uint32_t p = s ^ T.mask;
-            const uint64_t idx = (uint64_t)rank[p & right] + (uint64_t)offset[p >> ihf];
-            const double2 y = v1[idx];
-            const bool sel = __popc(s & T.selmask) & 1;
-            const double cr = sel ? T.c1r : T.c0r, ci = sel ? T.c1i : T.c0i;
-            ar = fma(cr, y.x, fma(-ci, y.y, ar));
-            ai = fma(cr, y.y, fma(ci, y.x, ai));
+    const uint64_t stride = (uint64_t)TPB * gridDim.x;
+    for (uint64_t i = (uint64_t)blockIdx.x * TPB + tid; i < dim; i += stride) {
+        const uint32_t s = list1[i];
+        const double2 x = v1[i];
+        double di = 0.0, dr;
+        if (REAL) {
+            dr = dg.c0r;
+            for (int g = 0; g < dg.ngroups; ++g) {
+                const uint32_t f = (dg.kind[g] == 0) ? (s & dg.mask[g]) : ((s ^ (s >> dg.shift[g])) & dg.mask[g]);
+                dr = fma((double)__popc(f), dg.wr[g], dr);
+            }
+        } else {
+            dr = sector_diag(dg, s, di);
         }
+        dr += shift;
+        double ar = dr * x.x, ai = dr * x.y;
+        if (!REAL) {
+            ar = dr * x.x - di * x.y;
+            ai = dr * x.y + di * x.x;
+        }
+        for (int t = 0; t < nterm; t += SEC_U) {
+            double2 y[SEC_U];
+#pragma unroll
+            for (int u = 0; u < SEC_U; ++u) {
+                const uint32_t m = terms[t + u].mask;   // (padded with zero masks: never active)
+                const uint32_t p = s ^ m;
+                y[u] = make_double2(0.0, 0.0);
+                if (__popc(s & m) == 1) {   // else the partner lies outside the sector: coefficient 0
+                    const uint32_t at = LDS ? off[p >> ihf] + rk[p & right] : offset[p >> ihf] + rank[p & right];
+                    y[u] = v1[at];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < SEC_U; ++u) {
+                // an active partner's selector is odd (see sector_terms): c1
+                const double cr = terms[t + u].c1r, ci = terms[t + u].c1i;
+                if (REAL) {
+                    ar = fma(cr, y[u].x, ar);
+                    ai = fma(cr, y[u].y, ai);
+                } else {
+                    ar = fma(cr, y[u].x, fma(-ci, y[u].y, ar));
+                    ai = fma(cr, y[u].y, fma(ci, y[u].x, ai));
+                }
+            }
+        }
+        ar *= x_s;
+        ai *= x_s;
         pr_re += x.x * ar + x.y * ai;
         pr_im += x.x * ai - x.y * ar;
-        double2 o;
-        if (fresh) {
-            o = make_double2(ar, ai);
-        } else {
-            const double2 old = v0[l];
-            o = make_double2(old.x + ar, old.y + ai);
+        double2 o = make_double2(ar, ai);
+        if (!fresh) {
+            const double2 old = v0[i];
+            o = make_double2(fma(y_s, old.x, ar), fma(y_s, old.y, ai));
         }
-        v0[l] = o;
+        v0[i] = o;
     }
-    const int tid = threadIdx.x;
     red[2 * tid] = pr_re;
     red[2 * tid + 1] = pr_im;
     __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
+    for (int st = TPB / 2; st > 0; st >>= 1) {
         if (tid < st) {
             red[2 * tid] += red[2 * (tid + st)];
             red[2 * tid + 1] += red[2 * (tid + st) + 1];
@@ -189,35 +235,64 @@ static int sector_terms(const S12Plan &pl, std::vector<SectorTerm> &out)
     return PNED_OK;
 }
 
+// device copy of the terms, padded to whole batches with terms that never apply
+static int upload_sector_terms(pned_ctx *ctx, std::vector<SectorTerm> st)
+{
+    ctx->sector_nterm = (int)st.size();
+    ctx->sector_real = (ctx->s12.c0i == 0.0) ? 1 : 0;
+    for (const SectorTerm &t : st)
+        if (t.c1i != 0.0) ctx->sector_real = 0;
+    for (const DiagGroup &g : ctx->s12.diag)
+        if (g.wi != 0.0) ctx->sector_real = 0;
+    st.resize((st.size() / SEC_U + 1) * SEC_U, SectorTerm{0, 0, 0.0, 0.0, 0.0, 0.0});
+    PNED_HIP(hipStreamSynchronize(ctx->stream));
+    if (ctx->d_sterms) PNED_HIP(hipFree(ctx->d_sterms));
+    ctx->d_sterms = nullptr;
+    PNED_HIP(hipMalloc(&ctx->d_sterms, sizeof(SectorTerm) * st.size()));
+    PNED_HIP(hipMemcpy(ctx->d_sterms, st.data(), sizeof(SectorTerm) * st.size(), hipMemcpyHostToDevice));
+    return PNED_OK;
+}
+
 int refresh_sector_terms(pned_ctx *ctx)
 {
     std::vector<SectorTerm> st;
     PNED_TRY(sector_terms(ctx->s12, st));
-    PNED_HIP(hipStreamSynchronize(ctx->stream));
-    if (ctx->d_sterms) PNED_HIP(hipFree(ctx->d_sterms));
-    ctx->d_sterms = nullptr;
-    PNED_HIP(hipMalloc(&ctx->d_sterms, sizeof(SectorTerm) * std::max<size_t>(st.size(), 1)));
-    if (!st.empty())
-        PNED_HIP(hipMemcpy(ctx->d_sterms, st.data(), sizeof(SectorTerm) * st.size(), hipMemcpyHostToDevice));
-    ctx->sector_nterm = (int)st.size();
-    return PNED_OK;
+    return upload_sector_terms(ctx, st);
 }
 
-int launch_hv_sector(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double eperbd, bool fresh, double *prdct_host)
+int launch_hv_sector(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double eperbd, bool fresh, double *prdct_host,
+                     const double *d_xs, const double *d_ys)
 {
     if (v1->nvec != 1 || v1->dtype != PNED_C128)
         return fail(PNED_E_UNSUPPORTED, "sector H.v takes one complex128 column");
     // the diagonal table is shared with the full-space path
     PNED_TRY(ensure_s12_plan(ctx, 0, PNED_C128));
     const uint64_t dim = (uint64_t)ctx->dim;
-    int grid = (int)std::min<uint64_t>((dim + 255) / 256, 4096);
+    const int ihf = (ctx->n + 1) / 2, ihf0 = ctx->n / 2;
+    // tables in LDS up to 28 sites (98 KB), from L2 above.  1024 threads share one copy from 2^19
+    // states on (N=24: 108 us a call, against 118-122 on 256 threads), on a grid of resident
+    // blocks that stage it once (512; 256-thread blocks in a partial second round took 152)
+    const size_t tab = (sizeof(uint32_t) << ihf0) + (sizeof(uint16_t) << ihf);
+    const bool lds = ihf <= 14;
+    const int tpb = lds && (ihf == 14 || dim >= (1u << 19)) ? 1024 : 256;
+    const uint64_t cap = tpb == 1024 ? 512 : 4096;
+    const int grid = (int)std::min<uint64_t>((dim + tpb - 1) / tpb, cap);
     PNED_TRY(ensure_partial(ctx, 2 * (size_t)grid));
     PNED_TRY(ensure_result(ctx, 8));
-    hipLaunchKernelGGL(hv_sector_kernel, dim3(grid), dim3(256), 0, ctx->stream, (const double2 *)v1->data,
-                       (double2 *)v0->data, ctx->d_list1, ctx->d_srank, ctx->d_soffset,
-                       (const SectorTerm *)ctx->d_sterms, ctx->sector_nterm, ctx->d_diag, (ctx->n + 1) / 2,
-                       -(double)ctx->ibond * eperbd, fresh ? 1 : 0, dim, ctx->d_partial);
-    PNED_HIP(hipGetLastError());
+    auto launch = [&](auto k) -> int {
+        PNED_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     (int)(lds ? tab : 0)));
+        hipLaunchKernelGGL(k, dim3(grid), dim3(tpb), lds ? tab : 0, ctx->stream, (const double2 *)v1->data,
+                           (double2 *)v0->data, ctx->d_list1, ctx->d_srank, ctx->d_soffset,
+                           (const SectorTerm *)ctx->d_sterms, ctx->sector_nterm, ctx->d_diag, ihf, ihf0,
+                           -(double)ctx->ibond * eperbd, fresh ? 1 : 0, dim, d_xs, d_ys, ctx->d_partial);
+        PNED_HIP(hipGetLastError());
+        return PNED_OK;
+    };
+    const bool real = ctx->sector_real != 0;
+    if (tpb == 1024) PNED_TRY(real ? launch(hv_sector_kernel<true, true, 1024>) : launch(hv_sector_kernel<false, true, 1024>));
+    else if (lds) PNED_TRY(real ? launch(hv_sector_kernel<true, true, 256>) : launch(hv_sector_kernel<false, true, 256>));
+    else PNED_TRY(real ? launch(hv_sector_kernel<true, false, 256>) : launch(hv_sector_kernel<false, false, 256>));
     PNED_TRY(reduce_rows_result(ctx, grid, 2));
     if (prdct_host) {
         PNED_HIP(hipMemcpyAsync(ctx->h_result, ctx->d_result, 2 * sizeof(double), hipMemcpyDeviceToHost,
@@ -282,14 +357,11 @@ extern "C" int pned_ctx_sz_sector(pned_ctx *ctx, int n_down)
     PNED_HIP(hipMalloc((void **)&ctx->d_list1, sizeof(uint32_t) * list1.size()));
     PNED_HIP(hipMalloc((void **)&ctx->d_srank, sizeof(uint32_t) * rank.size()));
     PNED_HIP(hipMalloc((void **)&ctx->d_soffset, sizeof(uint32_t) * offset.size()));
-    PNED_HIP(hipMalloc(&ctx->d_sterms, sizeof(SectorTerm) * std::max<size_t>(st.size(), 1)));
     PNED_HIP(hipMemcpy(ctx->d_list1, list1.data(), sizeof(uint32_t) * list1.size(), hipMemcpyHostToDevice));
     PNED_HIP(hipMemcpy(ctx->d_srank, rank.data(), sizeof(uint32_t) * rank.size(), hipMemcpyHostToDevice));
     PNED_HIP(hipMemcpy(ctx->d_soffset, offset.data(), sizeof(uint32_t) * offset.size(), hipMemcpyHostToDevice));
-    if (!st.empty())
-        PNED_HIP(hipMemcpy(ctx->d_sterms, st.data(), sizeof(SectorTerm) * st.size(), hipMemcpyHostToDevice));
+    PNED_TRY(upload_sector_terms(ctx, st));
     ctx->sector_k = n_down;
-    ctx->sector_nterm = (int)st.size();
     ctx->dim = (int64_t)total;
     return PNED_OK;
 }

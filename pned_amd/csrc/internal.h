@@ -245,6 +245,7 @@ struct pned_ctx {
     uint32_t *d_srank = nullptr;     // rank of a right half among its popcount class
     uint32_t *d_soffset = nullptr;   // first index of a left half's block
     void *d_sterms = nullptr;        // two-bit flip terms
+    int sector_real = 0;             // no imaginary part in its terms and diagonal
     double *d_colcoef = nullptr;     // batch contexts: per-column term coefficients
     double *d_coldiag = nullptr;     // batch contexts: per-column diagonal weights
     int pd_threads = -1;
@@ -322,8 +323,9 @@ int check_same_layout(const pned_vec *x, const pned_vec *y);
 int vec_to_host(const pned_vec *v, void *host, int64_t offset, int64_t count);
 int vec_from_host(pned_vec *v, const void *host, int64_t offset, int64_t count);
 // S^z sector basis: H.v and table release
+// (d_xs, d_ys: optional device factors, v0 = y v0 + H (x v1))
 int launch_hv_sector(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double eperbd, bool fresh,
-                     double *prdct_host);
+                     double *prdct_host, const double *d_xs = nullptr, const double *d_ys = nullptr);
 void free_sector(pned_ctx *ctx);
 // intalv_xy, S=1/2 sectors: v (sector k + ipm of ctx) = sum_j e^{i q.r_j} (x with bit j
 // set (ipm = +1) or cleared (-1)); x in sector k of x->ctx

@@ -18,14 +18,14 @@ double cabs2(const double *z) { return std::sqrt(z[0] * z[0] + z[1] * z[1]); }
 
 // The Lanczos recursion of lnc1z and dsflnc1z (Hybrid_TPS_Lanczos.f90:111-120,
 // Hybrid_TPS_DSF.f90:228-250): v1 <- (v0 - alpha v1)/beta, v0 <- -beta v1, then
-// v0 += H v1, alpha = Re <v1|H v1>, beta = |v0 - <v1|H v1> v1|.  In the S=1/2 full space
-// (and with the tiled spin-S kernel) the divisions by beta are left to the next H.v: x
+// v0 += H v1, alpha = Re <v1|H v1>, beta = |v0 - <v1|H v1> v1|.  For S=1/2 (full space and S^z
+// sectors) and with the tiled spin-S kernel the divisions by beta are left to the next H.v: x
 // holds v1/sx, the H.v input y is read times sy, and the two buffers swap roles each step,
 // so a step streams the vectors 3 times besides the H.v instead of 6.  Other bases run the
 // reference's update as written.
 // finish() leaves v1 and v0 as the reference's loop leaves them (the last Lanczos vector
 // and H v1 - beta v_prev), so a dump for restart holds the same vectors.
-// With graphs on (one S=1/2 full-space column), the steps are enqueued in their device form:
+// With graphs on (one S=1/2 column), the steps are enqueued in their device form:
 // each step forms its sx, sy from the previous step's beta^2 on the device and leaves
 // [prd, beta^2] in a history slot, so advance() replays 5 steps at a time from a captured
 // graph (one per buffer role) and reads the 5 slots back once.  The host repeats the same
@@ -47,8 +47,7 @@ struct LanczosSteps {
     LanczosSteps(pned_ctx *c, pned_vec *a, pned_vec *b, bool explicit_update = false)
         : ctx(c), v1(a), v0(b),
           lazy(!explicit_update && a->nvec == 1 &&
-               ((c->q == 2 && c->sector_k < 0) ||
-                (c->q >= 3 && c->q <= 5 && c->spin_tiled && a->dtype == PNED_C128))),
+               (c->q == 2 || (c->q >= 3 && c->q <= 5 && c->spin_tiled && a->dtype == PNED_C128))),
           dev(lazy && c->q == 2 && c->use_graphs),
           X(a), Y(b)
     {

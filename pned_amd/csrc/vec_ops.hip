@@ -881,8 +881,9 @@ int lanczos_lazy_step(pned_ctx *ctx, pned_vec *x, pned_vec *y, const double *sx,
     PNED_TRY(check_hv_pair(ctx, x, y));
     PNED_TRY(check_pow2_cols(x->nvec));
     const bool spin = ctx->q >= 3 && ctx->q <= 5 && ctx->spin_tiled;
-    if (!((ctx->q == 2 && ctx->sector_k < 0) || (spin && x->nvec == 1 && x->dtype == PNED_C128)))
-        return fail(PNED_E_UNSUPPORTED, "lazy Lanczos step: S=1/2 full space or the tiled spin-S kernel");
+    const bool sector = ctx->sector_k >= 0;
+    if (!(ctx->q == 2 || (spin && x->nvec == 1 && x->dtype == PNED_C128)))
+        return fail(PNED_E_UNSUPPORTED, "lazy Lanczos step: S=1/2 or the tiled spin-S kernel");
     const int nc = x->nvec;
     const size_t nelem = (size_t)x->dim * nc;
     const int grid = RED_GRID;
@@ -899,6 +900,8 @@ int lanczos_lazy_step(pned_ctx *ctx, pned_vec *x, pned_vec *y, const double *sx,
     bool fused = false;
     if (spin)
         PNED_TRY(launch_hv_spin_tiled(ctx, x, y, 0.0, fresh, nullptr, sx[0], fresh ? 1.0 : sy[0]));
+    else if (sector)
+        PNED_TRY(launch_hv_sector(ctx, x, y, 0.0, fresh, nullptr, d, fresh ? nullptr : d + nc));
     else
         PNED_TRY(launch_hv_s12(ctx, x, y, 0.0, fresh, nullptr, d, fresh ? nullptr : d + nc, &fused));
     if (fused) {   // the last pass formed y - Re(alpha) sx x and beta^2 already
@@ -973,12 +976,15 @@ int lanczos_lazy_setup(pned_ctx *ctx, const pned_vec *x, const pned_vec *y)
 int lanczos_lazy_enqueue(pned_ctx *ctx, pned_vec *x, pned_vec *y, bool fresh, double *st, double *slot)
 {
     PNED_TRY(check_hv_pair(ctx, x, y));
-    if (x->nvec != 1 || ctx->q != 2 || ctx->sector_k >= 0)
-        return fail(PNED_E_UNSUPPORTED, "captured Lanczos step: one column of an S=1/2 full-space context");
+    if (x->nvec != 1 || ctx->q != 2)
+        return fail(PNED_E_UNSUPPORTED, "captured Lanczos step: one column of an S=1/2 context");
     hipLaunchKernelGGL(k_lz_scale, dim3(1), dim3(64), 0, ctx->stream, st, fresh ? 1 : 0);
     PNED_HIP(hipGetLastError());
     bool fused = false;
-    PNED_TRY(launch_hv_s12(ctx, x, y, 0.0, fresh, nullptr, st, fresh ? nullptr : st + 1, &fused));
+    if (ctx->sector_k >= 0)
+        PNED_TRY(launch_hv_sector(ctx, x, y, 0.0, fresh, nullptr, st, fresh ? nullptr : st + 1));
+    else
+        PNED_TRY(launch_hv_s12(ctx, x, y, 0.0, fresh, nullptr, st, fresh ? nullptr : st + 1, &fused));
     if (!fused) {
         const size_t nelem = (size_t)x->dim;
         hipLaunchKernelGGL(k_copy_f64, dim3(1), dim3(64), 0, ctx->stream, ctx->d_result, st + 2, 2);
