@@ -692,6 +692,267 @@ __global__ __launch_bounds__(TPB, (TM_WAVES<Real, TPB, R>)) void hv_s12_tm(const
     }
 }
 
+// Short vectors: several workgroups per tile.  A pass of hv_s12_tm on a vector of a few tiles leaves
+// most of the chip idle and is one serial chain per tile (address tables, v1, LDS, a scalar-cache
+// miss and an LDS round trip per term and sweep, v0, the reduction).  Here every one of a tile's
+// `split` workgroups stages the whole tile in LDS and forms one state per thread: the states whose
+// low bits in the tile are the workgroup's number.  Addresses come from the bit positions in the
+// kernel arguments, v0 is loaded beside v1, and every term record is touched once while those
+// loads fly, so the term loop hits the scalar cache.  The states' values are those of hv_s12_tm and
+// so are the partial sums: 256 threads owning the tile would each sum their slots and then add in
+// halves from the top; a workgroup's states are whole such threads, equal in their low bits, so it
+// ends with the first halvings and reduce_split does the rest.
+// us per H.v with its reduction and read-back, hv_s12_tm on 256 threads -> here (field, complex128):
+// N=12 46.6 -> 30.0, N=16 43.5 -> 37.9, N=18 67 -> 59; 40 Lanczos steps at N=16 2.40 -> 2.02 ms.
+constexpr int SPLIT_ROUND = 8;
+struct SmallArgs {
+    int colbits, ncol;
+    int first_term, nreal, nterm;
+    int diag, fresh, lz_mode;
+    int K, lsplit;         // tile bits, log2 of the workgroups per tile
+    double shift;
+    const double *colscale, *yscale, *lz_prd;
+    uint64_t tb, tbt, tbh; // memory bits of the tile from its bit 0, lsplit and K - lsplit, 5 bits each
+    uint64_t ob;           // (an array would be indexed through scratch memory); of the tile number
+};
+
+template <typename Real>
+__global__ __launch_bounds__(1024) void hv_s12_split(const typename C2<Real>::T *__restrict__ v1,
+                                                     typename C2<Real>::T *__restrict__ v0,
+                                                     const TmTerm *__restrict__ terms,
+                                                     const DiagDev *__restrict__ diagp, SmallArgs a,
+                                                     double *__restrict__ partial)
+{
+    using V = typename C2<Real>::T;
+    using A = Real;
+    extern __shared__ unsigned char smem_raw[];
+    V *tile = reinterpret_cast<V *>(smem_raw);
+    const int tid = threadIdx.x, tpb = blockDim.x;   // tpb << lsplit = 2^K
+    const uint32_t sub = blockIdx.x & ((1u << a.lsplit) - 1u), tno = blockIdx.x >> a.lsplit;
+    // bit k of v to the k-th position (at most 12 bits; the positions above v's bits do not matter)
+    auto deposit = [](uint32_t v, uint64_t bits) {
+        uint32_t o = 0;
+        static_for<12>([&](auto k) { o |= ((v >> k) & 1u) << ((uint32_t)(bits >> (5 * k)) & 31u); });
+        return o;
+    };
+    const uint32_t ob = deposit(tno, a.ob);
+    const uint32_t j = ((uint32_t)tid << a.lsplit) | sub;   // this thread's state in the tile
+    const uint32_t at = ob | deposit(sub, a.tb) | deposit((uint32_t)tid, a.tbt);
+    const bool rd0 = !(a.diag && a.fresh) && a.lz_mode != 1;
+    V y{};
+    if (rd0) y = v0[at];
+    // the whole tile, SPLIT_ROUND states a thread at a time: tid's address, and the bits above the
+    // workgroup's size per round
+    const int rounds = 1 << a.lsplit;
+    const uint32_t a0 = ob | deposit((uint32_t)tid, a.tb);
+    Real sr[SPLIT_ROUND], si[SPLIT_ROUND];   // (components: a V[] array is not kept in registers)
+    auto fetch = [&](int g) {
+        static_for<SPLIT_ROUND>([&](auto I) {
+            if (g + I < rounds) {
+                const V t = v1[a0 | deposit((uint32_t)(g + I), a.tbh)];
+                sr[I] = t.x;
+                si[I] = t.y;
+            }
+        });
+    };
+    auto stage = [&](int g) {
+        static_for<SPLIT_ROUND>([&](auto I) {
+            if (g + I < rounds) {
+                V t;
+                t.x = sr[I];
+                t.y = si[I];
+                tile[tid + tpb * (g + I)] = t;
+            }
+        });
+    };
+    fetch(0);
+    const int col = (int)(j & (uint32_t)(a.ncol - 1));
+    const A colsc = a.colscale ? (A)a.colscale[col] : (A)1;
+    const A ys = (a.diag && a.yscale) ? (A)a.yscale[col] : (A)1;
+    double lar = 0.0, lai = 0.0;
+    if (a.lz_mode == 2) {
+        lar = (double)colsc * a.lz_prd[2 * col];
+        lai = (double)colsc * a.lz_prd[2 * col + 1];
+    }
+    const int dprog = a.diag ? diagp->nprog : 0;
+    const uint32_t dpa = dprog ? diagp->prog_a[tid & 63] : 0u;
+    const uint32_t dpb = dprog ? diagp->prog_b[tid & 63] : 0u;
+    {
+        uint32_t w = 0;
+#pragma unroll 8
+        for (int t = 0; t < a.nterm; ++t) w ^= terms[a.first_term + t].flags;
+        asm volatile("" ::"s"(w));
+    }
+    stage(0);
+    for (int g = SPLIT_ROUND; g < rounds; g += SPLIT_ROUND) {
+        fetch(g);
+        stage(g);
+    }
+    __syncthreads();
+    const V x = tile[j];
+
+    A ar = (A)0, ai = (A)0;
+    if (a.diag) {
+        const uint32_t st = (uint32_t)(at >> a.colbits);
+        double dr, di;
+        if (dprog) {   // the lane program (see DiagDev), the whole state at once
+            dr = diagp->c0r + a.shift;
+            di = diagp->c0i;
+            uint32_t cnt = 0u;
+            for (int e = 0; e < dprog; ++e) {
+                const uint32_t pa = (uint32_t)__builtin_amdgcn_readlane((int)dpa, e);
+                const uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)dpb, e);
+                cnt += (uint32_t)__popc(((pa & 64u) ? (st ^ (st >> (pa & 63u))) : st) & m);
+                if (pa & 128u) {
+                    const int c = (int)((pa >> 8) & 7u);
+                    const uint64_t wrb = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)dpa, 48 + c) |
+                                         ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)dpa, 56 + c) << 32);
+                    const uint64_t wib = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)dpb, 48 + c) |
+                                         ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)dpb, 56 + c) << 32);
+                    dr = fma((double)cnt, __longlong_as_double((long long)wrb), dr);
+                    di = fma((double)cnt, __longlong_as_double((long long)wib), di);
+                    cnt = 0u;
+                }
+            }
+        } else {
+            dr = diag_value_re(*diagp, st, di) + a.shift;
+        }
+        ar = (A)(dr * (double)x.x - di * (double)x.y);
+        ai = (A)(dr * (double)x.y + di * (double)x.x);
+    }
+
+    const uint32_t jb = j * (uint32_t)sizeof(V);
+    auto run = [&](int t, const int e, auto CXc) {
+        constexpr bool CX = decltype(CXc)::value;
+        // slot bits are kept whole: flip mask mlo | mhi, selector slo | shi (one thread per slot)
+        auto read = [&](const TmTerm &T) {
+            return *reinterpret_cast<const V *>(smem_raw + (jb ^ (T.mlo * (uint32_t)sizeof(V))));
+        };
+        auto add = [&](const TmTerm &T, const V &p) {
+            const bool f = (__popc(j & T.slo) + __popc(ob & (uint32_t)T.sout)) & 1;
+            const A c0r = (A)uniform(T.c0r), c1r = (A)uniform(T.c1r);
+            const A cr = f ? c1r : c0r;
+            ar = fma(cr, (A)p.x, ar);
+            if constexpr (CX) {
+                const A c0i = (A)uniform(T.c0i), c1i = (A)uniform(T.c1i);
+                const A ci = f ? c1i : c0i;
+                ar = fma(-ci, (A)p.y, ar);
+                ai = fma(cr, (A)p.y, ai);
+                ai = fma(ci, (A)p.x, ai);
+            } else {
+                ai = fma(cr, (A)p.y, ai);
+            }
+        };
+        for (; t + 3 < e; t += 4) {
+            const TmTerm T0 = terms[t], T1 = terms[t + 1], T2 = terms[t + 2], T3 = terms[t + 3];
+            const V p0 = read(T0), p1 = read(T1), p2 = read(T2), p3 = read(T3);
+            add(T0, p0);
+            add(T1, p1);
+            add(T2, p2);
+            add(T3, p3);
+        }
+        for (; t < e; ++t) {
+            const TmTerm T0 = terms[t];
+            add(T0, read(T0));
+        }
+    };
+    run(a.first_term, a.first_term + a.nreal, std::false_type{});
+    run(a.first_term + a.nreal, a.first_term + a.nterm, std::true_type{});
+
+    if (a.colscale) {
+        ar *= colsc;
+        ai *= colsc;
+    }
+    double2 *cs = reinterpret_cast<double2 *>(smem_raw + (sizeof(V) << a.K));   // for the partial sums
+    if (a.lz_mode == 2) {
+        const double wr0 = (double)fma(ys, (A)y.x, ar);
+        const double wi0 = (double)fma(ys, (A)y.y, ai);
+        const double xr_ = (double)x.x * (double)colsc, xi_ = (double)x.y * (double)colsc;
+        // (rounded as hv_s12_tm's expressions are contracted)
+        const double wr = wr0 - fma(lar, xr_, -(lai * xi_));
+        const double wi = wi0 - fma(lai, xr_, lar * xi_);
+        cs[tid] = make_double2(wr, wi);
+        ar = (A)fma(-lar, xr_, wr0);
+        ai = (A)fma(-lar, xi_, wi0);
+    } else {
+        cs[tid] = make_double2((double)ar, (double)ai);
+        if (rd0) {
+            ar = fma(ys, (A)y.x, ar);
+            ai = fma(ys, (A)y.y, ai);
+        }
+    }
+    if (a.lz_mode != 1) {
+        V o;
+        o.x = (Real)ar;
+        o.y = (Real)ai;
+        v0[at] = o;
+    }
+    __syncthreads();
+    // slot j belongs to thread j mod 256 of the 256: here nv of them, slots nv apart in tid
+    const int nv = 256 >> a.lsplit, nr = tpb / nv;
+    double2 *red = cs + tpb;
+    if (tid < nv) {
+        double pr_re = 0.0, pr_im = 0.0;
+        for (int r = 0; r < nr; ++r) {
+            const double2 c = cs[tid + nv * r];
+            if (a.lz_mode == 2) {
+                pr_re = fma(c.x, c.x, fma(c.y, c.y, pr_re));
+            } else {
+                const V z = tile[((uint32_t)(tid + nv * r) << a.lsplit) | sub];
+                const double hr = c.x, hi = c.y;
+                pr_re += (double)z.x * hr + (double)z.y * hi;
+                pr_im += (double)z.x * hi - (double)z.y * hr;
+            }
+        }
+        red[tid] = make_double2(pr_re, pr_im);
+    }
+    __syncthreads();
+    // halvings while the partner is here and of the same column
+    const int keep = max(a.ncol >> a.lsplit, 1);
+    for (int s = nv / 2; s >= keep; s >>= 1) {
+        if (tid < s) {
+            red[tid].x += red[tid + s].x;
+            red[tid].y += red[tid + s].y;
+        }
+        __syncthreads();
+    }
+    if (tid < keep) {   // row tno: [sums still to be halved][column]
+        const size_t o = (size_t)tno * max(a.ncol, 1 << a.lsplit) + ((size_t)tid << a.lsplit) + sub;
+        partial[2 * o] = red[tid].x;
+        partial[2 * o + 1] = red[tid].y;
+    }
+}
+
+// the sums of hv_s12_split's rows: each row's `width` values are halved down to ncol columns, then the
+// rows are added as reduce_partials adds them
+__global__ __launch_bounds__(256) void reduce_split(const double *__restrict__ partial, int nrows, int ncol, int width,
+                                                    double *__restrict__ out)
+{
+    __shared__ double red[256];
+    const int c = blockIdx.x >> 1, part = blockIdx.x & 1, tid = threadIdx.x;
+    double s = 0.0;
+    for (int b = tid; b < nrows; b += 256) {
+        const double *row = partial + (size_t)b * 2 * width + part;
+        double v[16];
+        const int m = width / ncol;   // at most 16
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = i < m ? row[2 * (c + ncol * i)] : 0.0;
+#pragma unroll
+        for (int h = 8; h > 0; h >>= 1)
+            if (h < m)
+#pragma unroll
+                for (int i = 0; i < h; ++i) v[i] += v[i + h];
+        s += v[0];
+    }
+    red[tid] = s;
+    __syncthreads();
+    for (int k = 128; k > 0; k >>= 1) {
+        if (tid < k) red[tid] += red[tid + k];
+        __syncthreads();
+    }
+    if (tid == 0) out[blockIdx.x] = red[0];
+}
+
 // out[c] = sum over rows of partial[row][c]: one block per column, fixed strides and a
 // fixed tree, so the result is the same for the same partials
 __global__ __launch_bounds__(256) void reduce_partials(const double *__restrict__ partial, int nrows, int ncol2,
@@ -807,6 +1068,39 @@ static int dispatch_tm(pned_ctx *ctx, int TPB, int R, const void *v1, void *v0, 
     return fail(PNED_E_UNSUPPORTED, "no term-major H.v kernel instance for this tile shape");
 }
 
+template <typename Real>
+static int launch_split(pned_ctx *ctx, const void *v1, void *v0, const TmTerm *tm, const SmallArgs &a, double *partial,
+                        int tiles)
+{
+    using V = typename C2<Real>::T;
+    const int tpb = 1 << (a.K - a.lsplit);
+    const size_t lds = (sizeof(V) << a.K) + sizeof(double2) * ((size_t)tpb + 256);
+    auto kern = hv_s12_split<Real>;
+    PNED_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kern, dim3(tiles << a.lsplit), dim3(tpb), lds, ctx->stream, (const V *)v1, (V *)v0, tm,
+                       ctx->d_diag, a, partial);
+    PNED_HIP(hipGetLastError());
+    return PNED_OK;
+}
+
+// log2 of hv_s12_split's workgroups per tile, or -1 where a plan stays with hv_s12_tm: an untuned plan,
+// one operator, tiles of 2^8 .. 2^12 states (2^13 complex64 ones), at most 2^17 elements, or 2^18 in one complex128 column
+// (above, staging a tile several times costs more than the chain: 2^18 complex64 elements 49.6
+// against 47 us per H.v, 2^19 in 8 complex128 columns 79 against 64).  Workgroups of 1024 threads where that makes 256 or more of them, else smaller ones,
+// down to 256 threads
+static int split_plan(const pned_ctx *ctx, const S12Plan &pl, int colbits, bool c128)
+{
+    if (ctx->s12_kernel != 1 || pl.nop > 1 || ctx->tune_threads > 0 || ctx->tune_tile_bits > 0) return -1;
+    if (ctx->n + colbits > (c128 && colbits == 0 ? 18 : 17) || pl.passes.empty()) return -1;
+    const int K = pl.passes[0].K;
+    for (const PassPlan &pp : pl.passes)
+        if (pp.K != K || K < 8 || K > (c128 ? 12 : 13) || pp.ob.size() > 10) return -1;
+    int ls = std::max(0, K - 10);
+    const int tiles = (int)pl.passes[0].ob.size();
+    while (tiles + ls < 8 && ls < 4 && K - ls > 8) ++ls;
+    return ls;
+}
+
 // Tile-coordinate term table of one pass (see TmTerm), sorted into the term-major
 // kernel's categories: 0 real, 1 real with register selector bits, 2 complex, 3 complex
 // with register selector bits (batch contexts: every term complex).  ncat gets the counts.
@@ -907,21 +1201,17 @@ static int contiguous_bits(const std::vector<int> &b)
 }
 
 // Threads of the untuned term-major plan, by its tile size (complex128 figures: one column with
-// field, us per H.v).  Up to 2^18 elements 256 threads: other counts sum <v1|H v1> in another
-// order, and a Lanczos run over such short vectors amplifies the last bit (2^16 states, 40 steps:
-// to 1e-7).  2^12-state tiles 1024 threads up to 2^21 elements (N=20 57.9, on 512 68), 512 above
-// (N=24 533 against 565: two blocks per CU), but 1024 in batches (N=20 with 8 columns 277 against
-// 344).  2^13 1024 (N=28 9.08 ms, on 512 13.9).  complex64: 2^12 512 (N=24 383, on 1024 472), 2^13
-// 1024 (N=28 5.8 ms), 2^14 512 (1024 spill; N=24 with 64 columns 28.7 against 31.7 ms).
+// field, us per H.v).  2^12-state tiles 1024 threads up to 2^21 elements (N=20 57.9, on 512 68), 512
+// above (N=24 533 against 565: two blocks per CU), but 1024 in batches (N=20 with 8 columns 277
+// against 344).  2^13 1024 (N=28 9.08 ms, on 512 13.9).  complex64: 2^12 512 (N=24 383, on 1024 472),
+// 2^13 1024 (N=28 5.8 ms), 2^14 512 (1024 spill; N=24 with 64 columns 28.7 against 31.7 ms).
 static int default_threads(const pned_ctx *ctx, const S12Plan &pl, int colbits, bool c128)
 {
     const int K = pl.passes.empty() ? 12 : pl.passes[0].K;
-    const double elems = (double)ctx->dim * (double)(1ull << colbits);
-    // one tile in all: its block is all there is to sum (2^12 states: 46 us on 256, 34 on 1024)
-    if (K <= 11 || (elems <= (double)(1ull << 18) && K < ctx->n + colbits)) return 256;
+    const bool big = (double)ctx->dim * (double)(1ull << colbits) > (double)(1ull << 21);
+    if (K <= 11) return 256;
     if (!c128) return K == 13 ? 1024 : 512;
-    if (K == 12 && elems > (double)(1ull << 21) && colbits == 0) return 512;
-    return 1024;
+    return K == 12 && big && colbits == 0 ? 512 : 1024;
 }
 
 // the thread count whose register slots order a pass's terms (see build_tm_terms)
@@ -995,7 +1285,10 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
     const bool c128 = v1->dtype == PNED_C128;
     const size_t esz = c128 ? 16 : 8;
     // per-pass address tables (rebuilt when the plan or the thread count changes)
-    const int TPBpref = (ctx->tune_threads == 256 || ctx->tune_threads == 512 || ctx->tune_threads == 1024)
+    const int lsplit = split_plan(ctx, pl, colbits, c128);
+    const bool small = lsplit >= 0;
+    // (hv_s12_split keeps a slot's bits whole, as a table for 2^13 threads would)
+    const int TPBpref = small ? 8192 : (ctx->tune_threads == 256 || ctx->tune_threads == 512 || ctx->tune_threads == 1024)
                             ? ctx->tune_threads
                             : (ctx->s12_kernel == 1 ? default_threads(ctx, pl, colbits, c128) : 512);
     std::vector<int> tpb(npass), rr(npass);
@@ -1016,6 +1309,7 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
             const PassPlan &pp = pl.passes[p];
             PassDev &d = host[p];
             std::memset(&d, 0, sizeof(PassDev));
+            if (small) continue;   // (no address tables)
             const int LT = __builtin_ctz(tpb[p]);
             for (int t = 0; t < tpb[p]; ++t) {
                 uint64_t o = 0;
@@ -1063,7 +1357,7 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
         // the diagonal pass's lane program split by that pass's register bits
         if (ctx->d_diag_tm) PNED_HIP(hipFree(ctx->d_diag_tm));
         ctx->d_diag_tm = nullptr;
-        for (int p = 0; p < npass && pl.nop <= 1 && ctx->diag_host.nprog > 0; ++p) {
+        for (int p = 0; p < npass && !small && pl.nop <= 1 && ctx->diag_host.nprog > 0; ++p) {
             const PassPlan &pp = pl.passes[p];
             if (!pp.diag) continue;
             uint32_t slot_bits = 0;
@@ -1084,6 +1378,7 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
     // and 256 by about 0.5 ms
     auto pass_grid = [&](int p) {
         const uint64_t tc = 1ull << pl.passes[p].ob.size();
+        if (small) return (int)tc;   // at most 2^10, times 2^lsplit <= 4 or 16 workgroups
         const uint64_t fill = (tpb[p] <= 512 && esz << pl.passes[p].K <= LDS_LIMIT / 2) ? 512 : 256;
         const uint64_t want = std::max<uint64_t>(fill, tc / 8);
         return (int)std::min<uint64_t>(std::min<uint64_t>(tc, want), (uint64_t)grid_cap);
@@ -1091,6 +1386,17 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
     // partial rows: per column group [pass][block] of 2 ncol_t values, the groups one after another
     int rows_grp = 0;
     for (int p = 0; p < npass; ++p) rows_grp += pass_grid(p);
+    // values per partial row and column part, and the sum over rows
+    const int width = small ? std::max(ncol_t, 1 << lsplit) : ncol_t;
+    auto reduce_rows_of = [&](const double *part, int rows, double *out) -> int {
+        if (small)
+            hipLaunchKernelGGL(reduce_split, dim3(2 * ncol_t), dim3(256), 0, ctx->stream, part, rows, ncol_t, width, out);
+        else
+            hipLaunchKernelGGL(reduce_partials, dim3(2 * ncol_t), dim3(256), 0, ctx->stream, part, rows, 2 * ncol_t, out,
+                               0);
+        PNED_HIP(hipGetLastError());
+        return PNED_OK;
+    };
     // the non-temporal streams (see hv_s12_tm): whole 128-byte lines only
     const size_t vec_bytes = esz * (size_t)ctx->dim * (size_t)nvec;
     const int lowrun = pl.passes.empty() ? 0 : contiguous_bits(pl.passes[0].tb);
@@ -1123,27 +1429,51 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
         const int grid = pass_grid(p);
         const PassDev *pdp = reinterpret_cast<const PassDev *>(ctx->pd_dev) + p;
         const size_t tile_bytes = esz * (size_t)TPB * R;
+        SmallArgs sm{};
+        if (small) {
+            sm.colbits = colbits;
+            sm.ncol = ncol_t;
+            sm.first_term = a.first_term;
+            sm.nreal = a.ncat[0] + a.ncat[1];
+            sm.nterm = a.nterm;
+            sm.diag = a.diag;
+            sm.fresh = a.fresh;
+            sm.K = pp.K;
+            sm.lsplit = lsplit;
+            sm.shift = a.shift;
+            auto from = [&](int k0) {   // twelve positions are more than deposit() is ever given bits for
+                uint64_t w = 0;
+                for (int k = k0; k < pp.K && k < k0 + 12; ++k) w |= (uint64_t)expand(pp.tb[k]) << (5 * (k - k0));
+                return w;
+            };
+            sm.tb = from(0);
+            sm.tbt = from(lsplit);
+            sm.tbh = from(pp.K - lsplit);
+            for (int k = 0; k < a.nouter; ++k) sm.ob |= (uint64_t)expand(pp.ob[k]) << (5 * k);
+        }
         const bool tm = ctx->s12_kernel == 1 && (c128 ? has_tm<double>(TPB, R) : has_tm<float>(TPB, R)) &&
                         tile_bytes + tm_coef_bytes(a) <= LDS_LIMIT;
         const DiagDev *dgp = (pp.diag && ctx->d_diag_tm) ? ctx->d_diag_tm : ctx->d_diag;
-        if (!noalloc && lz_fused && p == npass - 1 && p > 0 && tm && c128 && nvec == 1 && pl.nop <= 1) {
+        if (!noalloc && lz_fused && p == npass - 1 && p > 0 && (tm || small) && c128 && nvec == 1 && pl.nop <= 1) {
             // deferred-normalisation Lanczos step: this pass's <v1|H v1> share first (no v0
             // traffic), alpha from all passes on the device, then the pass itself forms
             // v0 - Re(alpha) s v1 and the partials of beta^2
-            double *part = part_base + (size_t)total_rows * 2 * nvec;
-            a.lz_mode = 1;
-            PNED_TRY(dispatch_tm<double>(ctx, TPB, R, v1->data, v0->data, ctx->d_tm, dgp, pdp, a, part, grid));
+            double *part = part_base + (size_t)total_rows * 2 * width;
+            auto pass = [&](int mode) -> int {
+                a.lz_mode = sm.lz_mode = mode;
+                sm.lz_prd = a.lz_prd;
+                sm.colscale = a.colscale;
+                sm.yscale = a.yscale;
+                if (small) return launch_split<double>(ctx, v1->data, v0->data, ctx->d_tm, sm, part, grid);
+                return dispatch_tm<double>(ctx, TPB, R, v1->data, v0->data, ctx->d_tm, dgp, pdp, a, part, grid);
+            };
+            PNED_TRY(pass(1));
             total_rows += grid;
-            hipLaunchKernelGGL(reduce_partials, dim3(2 * nvec), dim3(256), 0, ctx->stream, ctx->d_partial, total_rows,
-                               2 * nvec, ctx->d_result, 0);
-            PNED_HIP(hipGetLastError());
-            a.lz_mode = 2;
+            PNED_TRY(reduce_rows_of(ctx->d_partial, total_rows, ctx->d_result));
             a.lz_prd = ctx->d_result;
-            part = ctx->d_partial + (size_t)total_rows * 2 * nvec;
-            PNED_TRY(dispatch_tm<double>(ctx, TPB, R, v1->data, v0->data, ctx->d_tm, dgp, pdp, a, part, grid));
-            hipLaunchKernelGGL(reduce_partials, dim3(2 * nvec), dim3(256), 0, ctx->stream, part, grid, 2 * nvec,
-                               ctx->d_result + 2 * nvec, 0);
-            PNED_HIP(hipGetLastError());
+            part = ctx->d_partial + (size_t)total_rows * 2 * width;
+            PNED_TRY(pass(2));
+            PNED_TRY(reduce_rows_of(part, grid, ctx->d_result + 2 * nvec));
             *lz_fused = true;
             return PNED_OK;
         }
@@ -1154,9 +1484,16 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
             void *y = static_cast<char *>(v0->data) + eo;
             a.colscale = d_colscale ? d_colscale + (size_t)g * ncol_t : nullptr;
             a.yscale = d_yscale ? d_yscale + (size_t)g * ncol_t : nullptr;
-            double *part = part_base + ((size_t)g * rows_grp + total_rows) * 2 * ncol_t;
+            double *part = part_base + ((size_t)g * rows_grp + total_rows) * 2 * width;
             int rc;
-            if (tm) {
+            if (small) {
+                sm.colscale = a.colscale;
+                sm.yscale = a.yscale;
+                if (c128)
+                    rc = launch_split<double>(ctx, x, y, ctx->d_tm, sm, part, grid);
+                else
+                    rc = launch_split<float>(ctx, x, y, ctx->d_tm, sm, part, grid);
+            } else if (tm) {
                 // the term table is in pass order, so the kernel indexes it by first_term as well
                 if (c128)
                     rc = dispatch_tm<double>(ctx, TPB, R, x, y, ctx->d_tm, dgp, pdp, a, part, grid);
@@ -1173,12 +1510,8 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
     }
     const int ncol2 = 2 * nvec;
     double *const out = noalloc ? result_ext : ctx->d_result;
-    for (int g = 0; g < ngrp; ++g) {
-        hipLaunchKernelGGL(reduce_partials, dim3(2 * ncol_t), dim3(256), 0, ctx->stream,
-                           part_base + (size_t)g * rows_grp * 2 * ncol_t, rows_grp, 2 * ncol_t,
-                           out + (size_t)g * 2 * ncol_t, 0);
-        PNED_HIP(hipGetLastError());
-    }
+    for (int g = 0; g < ngrp; ++g)
+        PNED_TRY(reduce_rows_of(part_base + (size_t)g * rows_grp * 2 * width, rows_grp, out + (size_t)g * 2 * ncol_t));
     if (noalloc) return PNED_OK;
     if (prdct_host) {
         PNED_HIP(hipMemcpyAsync(ctx->h_result, ctx->d_result, sizeof(double) * ncol2,

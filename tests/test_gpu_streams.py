@@ -30,3 +30,27 @@ def test_untuned_plan_matches_state_major(spec, cols, dtype):
     nd = np.sqrt(np.atleast_1d(ctx.calc_vec_inprdct(a, a)).real)
     assert np.all(nd <= tol * nb), (nd, nb)
     assert np.all(np.abs(pa - pb) <= tol * nb)   # |<x|Hx>| <= |Hx| for the unit x
+
+
+# hv_s12_split (short vectors, untuned) against hv_s12_tm on 256 threads: the same values and sums bit
+# for bit.  One tile and several, more and fewer columns than workgroups per tile, 256 and 1024 threads
+@pytest.mark.parametrize("spec,cols,dtype", [("2x2", 1, gpu.C128), ("2x2", 64, gpu.C64), ("2x3", 1, gpu.C64),
+                                             ("2x3", 16, gpu.C64), ("2x3", 32, gpu.C128), ("2x4", 1, gpu.C128),
+                                             ("2x4", 2, gpu.C64), (18, 1, gpu.C128)])
+def test_split_matches_tiles(spec, cols, dtype):
+    cl = lattice.get_cluster(spec)
+    got = []
+    for threads in (0, 256):
+        ctx = gpu.Context(model.build_operator(cl, 20, 126.0, field=0.1))
+        if threads:
+            ctx.tune(0, 0, threads)
+        x, y = ctx.vector(cols, dtype), ctx.vector(cols, dtype)
+        ctx.set_initial_vec(x, 5)
+        ctx.set_initial_vec(y, 6)
+        out = [np.atleast_1d(ctx.p_mltply_v3(x, y, 0.03)), y.download()]
+        if cols == 1 and dtype == gpu.C128:
+            _, a, b, _ = ctx.lnc1(x, y, fixed_steps=9, nvec=1)
+            out += [a, b, x.download(), y.download()]
+        got.append(out)
+    for p, q in zip(*got):
+        assert np.array_equal(p, q)
