@@ -242,6 +242,7 @@ constexpr int SP_MAX_BOND = 64;       // bonds per pass: one record per lane of 
 constexpr int SP_BASE_TAB = 4096;
 constexpr int SP_MAX_QQ = 25;         // q <= 5
 constexpr int SP_MAX_CLS = 64;        // off-diagonal (bond, partner shift) classes per pass: one per lane
+constexpr int SP_GRID_CAP = 2048;      // blocks per pass at most
 constexpr int SP_MAX_COEF = SP_MAX_CLS * SP_MAX_QQ;
 
 struct SpinPassDev {
@@ -467,6 +468,203 @@ __global__ __launch_bounds__(TPB) void hv_spin_pass(const double2 *__restrict__ 
     }
 }
 
+// One tile computed by several blocks, for passes whose tiles alone leave compute units idle
+// (spin 1, 12 sites: 81 tiles of 3^8 states on 256 units, one of which took two).  Each block
+// stages the whole tile and computes the register slots of its part, one tile a block.
+//
+// Register slots are the digits of the tile's top NR sites: slot r of the thread with lane
+// digits t holds the state t + LT r (LT = q^(K-NR), R = q^NR), so a slot's own digits are
+// uniform and a bond whose two sites are both lane digits has one coefficient for the S
+// slots of a thread.  The class loop is bound by LDS reads (16 bytes a lane for each partner),
+// and the rest is one serial chain: address tables, v1, barrier, classes, v0.
+// us per H.v with its read-back, hv_spin_pass -> this: spin 1 on 8 sites 60 -> 30, on 12 sites
+// 140 -> 66; 5 states a site, 8 sites 86 -> 70.
+template <int Q, int NR, int TPB, int S, bool CPLX>
+__global__ __launch_bounds__(TPB) void hv_spin_split(const double2 *__restrict__ v1, double2 *__restrict__ v0,
+                                                     const SpinPassDev *__restrict__ pd, SpinPassArgs a,
+                                                     double *__restrict__ partial)
+{
+    constexpr int QQ = Q * Q;
+    constexpr int R = (NR == 2) ? QQ : Q;
+    constexpr int PARTS = R / S;
+    constexpr int CW = CPLX ? 16 : 8;     // bytes per staged coefficient
+    static_assert(R % S == 0, "parts must tile the register slots");
+    extern __shared__ unsigned char spin_smem[];
+    double2 *tile = reinterpret_cast<double2 *>(spin_smem);
+    double2 *dg = tile + a.tsz;                                        // bond diagonals, shift included
+    unsigned char *cfb = reinterpret_cast<unsigned char *>(dg + a.nbond * QQ);   // class coefficients
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int LT = a.tsz / R;             // active threads
+    const bool act = tid < LT;
+    const int tl = min(tid, LT - 1);      // (the others repeat the last one's slots and store nothing)
+
+    // parts of a tile and neighbouring tiles on one XCD (blockIdx mod 8)
+    const uint32_t xc = blockIdx.x & 7u, per = gridDim.x >> 3, rem = gridDim.x & 7u;
+    const uint32_t item = xc * per + min(xc, rem) + (blockIdx.x >> 3);
+    const uint32_t tix = item / PARTS;
+    const int r0 = (int)(item % PARTS) * S;
+    const uint64_t base = pd->blo[tix % (uint32_t)a.nlo_mod] + pd->bhi[tix / (uint32_t)a.nlo_mod];
+    const uint32_t offl = pd->off[tl];
+    auto addr = [&](int r) { return base + pd->off[LT * r] + offl; };
+    {
+        double2 x[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) x[r] = v1[addr(r)];
+        for (int i = tid; i < a.nbond * QQ; i += TPB)
+            dg[i] = make_double2(pd->diag[2 * i] + (pd->diag_kept[i] ? a.shift : 0.0), pd->diag[2 * i + 1]);
+        const int ncoef = a.ncls * QQ;
+        double *cf = reinterpret_cast<double *>(cfb);
+        for (int i = tid; i < ncoef; i += TPB) {
+            if (CPLX) {
+                cf[2 * i] = pd->cls_c[2 * i];
+                cf[2 * i + 1] = pd->cls_c[2 * i + 1];
+            } else {
+                cf[i] = pd->cls_c[2 * i];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (act) tile[tid + LT * r] = x[r];
+    }
+    // the pass's bond and class records, lane b / c of every wave
+    const int brec = (lane < a.nbond) ? pd->bond_rec[lane] : 0;
+    const int crec = (lane < a.ncls) ? pd->cls_delta[lane] : 0;
+    const bool rd0 = !(a.diag_first && a.fresh);
+    const double ysc = a.diag_first ? a.ys : 1.0;
+    const uint32_t tmax = (uint32_t)(a.tsz - 1) * 16u;
+    double2 y[S];
+#pragma unroll
+    for (int u = 0; u < S; ++u) y[u] = rd0 ? v0[addr(r0 + u)] : make_double2(0.0, 0.0);
+    // digit words, 4 bits per tile digit: the thread's lane digits, and slot r's own
+    uint32_t dw = 0;
+    {
+        int x = tl;
+        for (int k = 0; k < a.K - NR; ++k) {
+            dw |= (uint32_t)(x % Q) << (4 * k);
+            x /= Q;
+        }
+    }
+    const int rsh = 4 * (a.K - NR);
+    uint32_t rw[S];
+#pragma unroll
+    for (int u = 0; u < S; ++u) {
+        const int r = r0 + u;
+        rw[u] = (uint32_t)(r % Q) << rsh | (NR == 2 ? (uint32_t)(r / Q) << (rsh + 4) : 0u);
+    }
+    // output local state of a bond with digit-word shifts sa (min site), sb (max site)
+    auto local = [&](uint32_t w, int sa, int sb) { return Q * (int)((w >> sb) & 15u) + (int)((w >> sa) & 15u); };
+    __syncthreads();
+
+    double ar[S], ai[S];
+    uint32_t jb[S];   // byte offset of the slot's state in the tile
+#pragma unroll
+    for (int u = 0; u < S; ++u) {
+        jb[u] = (uint32_t)(tl + LT * (r0 + u)) * 16u;
+        double sr = 0.0, si = 0.0;
+        if (CPLX && a.diag_first) si = a.zi;
+        for (int b = 0; b < a.nbond; ++b) {
+            const int rec = __builtin_amdgcn_readlane(brec, b);
+            const int sa = rec & 31, sb = (rec >> 5) & 31;
+            const double2 g = dg[b * QQ + local(dw, sa, sb) + local(rw[u], sa, sb)];
+            sr += g.x;
+            si += g.y;
+        }
+        if (a.diag_first) sr += a.zr;
+        // a real pass: only the complex diagonal shift of pass 0 has an imaginary part
+        if (!CPLX) si = a.diag_first ? a.zi : 0.0;
+        const double2 x = *reinterpret_cast<const double2 *>(spin_smem + jb[u]);
+        ar[u] = fma(sr, x.x, -si * x.y);
+        ai[u] = fma(sr, x.y, si * x.x);
+    }
+#pragma unroll 1
+    for (int b = 0; b < a.nbond; ++b) {
+        const int rec = __builtin_amdgcn_readlane(brec, b);
+        const int sa = rec & 31, sb = (rec >> 5) & 31;
+        const int c0 = (rec >> 10) & 63, c1 = (rec >> 16) & 127;
+        const unsigned char *cl = cfb + (size_t)(local(dw, sa, sb) * CW);
+        int orr[S];   // the slot's part of the output local state, in bytes
+#pragma unroll
+        for (int u = 0; u < S; ++u) orr[u] = local(rw[u], sa, sb) * CW;
+        // N classes from c on, all of their reads before the first use; ONE: one coefficient
+        // for the thread's slots
+        auto classes = [&](int c, auto N, auto ONE) {
+            double2 p[N * S], cc[ONE ? N : N * S];
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                const uint32_t dl = (uint32_t)__builtin_amdgcn_readlane(crec, c + k);
+                const unsigned char *ck = cl + (size_t)(c + k) * QQ * CW;
+#pragma unroll
+                for (int u = 0; u < S; ++u) {
+                    // a partner beyond the tile has coefficient 0: its offset is clamped
+                    p[k * S + u] = *reinterpret_cast<const double2 *>(spin_smem + min(jb[u] + dl, tmax));
+                    if (ONE && u > 0) continue;
+                    const unsigned char *cp = ONE ? ck : ck + orr[u];
+                    double2 &c1 = cc[ONE ? k : k * S + u];
+                    if (CPLX) c1 = *reinterpret_cast<const double2 *>(cp);
+                    else c1.x = *reinterpret_cast<const double *>(cp);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < N; ++k)
+#pragma unroll
+                for (int u = 0; u < S; ++u) {
+                    const double2 &c1 = cc[ONE ? k : k * S + u], &q = p[k * S + u];
+                    if (CPLX) {
+                        ar[u] = fma(c1.x, q.x, fma(-c1.y, q.y, ar[u]));
+                        ai[u] = fma(c1.x, q.y, fma(c1.y, q.x, ai[u]));
+                    } else {
+                        ar[u] = fma(c1.x, q.x, ar[u]);
+                        ai[u] = fma(c1.x, q.y, ai[u]);
+                    }
+                }
+        };
+        using N1 = std::integral_constant<int, 1>;
+        using N2 = std::integral_constant<int, 2>;
+        int c = c0;
+        if (sa < rsh && sb < rsh) {
+#pragma unroll 1
+            for (; c + 2 <= c1; c += 2) classes(c, N2{}, std::true_type{});
+            if (c < c1) classes(c, N1{}, std::true_type{});
+        } else {
+#pragma unroll 1
+            for (; c + 2 <= c1; c += 2) classes(c, N2{}, std::false_type{});
+            if (c < c1) classes(c, N1{}, std::false_type{});
+        }
+    }
+    double pr_re = 0.0, pr_im = 0.0;
+#pragma unroll
+    for (int u = 0; u < S; ++u) {
+        if (!act) continue;
+        const double2 x = *reinterpret_cast<const double2 *>(spin_smem + jb[u]);
+        const double hr = ar[u] * a.xs, hi = ai[u] * a.xs;
+        if (a.dotu) {
+            pr_re += x.x * hr - x.y * hi;
+            pr_im += x.x * hi + x.y * hr;
+        } else {
+            pr_re += x.x * hr + x.y * hi;
+            pr_im += x.x * hi - x.y * hr;
+        }
+        v0[addr(r0 + u)] = make_double2(fma(ysc, y[u].x, hr), fma(ysc, y[u].y, hi));
+    }
+    // sum over the lanes of each wave, then over the waves
+    for (int st = 32; st > 0; st >>= 1) {
+        pr_re += __shfl_down(pr_re, st);
+        pr_im += __shfl_down(pr_im, st);
+    }
+    __syncthreads();   // the diagonals are no longer read
+    if (lane == 0) dg[tid >> 6] = make_double2(pr_re, pr_im);
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < TPB / 64; ++w) {
+            pr_re += dg[w].x;
+            pr_im += dg[w].y;
+        }
+        partial[2 * blockIdx.x] = pr_re;
+        partial[2 * blockIdx.x + 1] = pr_im;
+    }
+}
+
 // ---- planner (host only) ------------------------------------------------------------
 
 namespace {
@@ -597,7 +795,11 @@ std::vector<std::vector<int>> spin_cover(int n, const std::vector<int32_t> &sp, 
     auto best = spin_greedy_cover(n, sp, ibond, K, L);
     if (best.empty()) return best;
     uint64_t seed = SPIN_COVER_SEED ^ ((uint64_t)K << 8) ^ (uint64_t)L;
-    for (int P = (int)best.size() - 1; P >= 1; --P) {
+    // every site with a bond is in some set: no search where the free places are too few
+    std::vector<char> bonded(n, 0);
+    for (int b = 0; b < ibond; ++b) bonded[sp[2 * b]] = bonded[sp[2 * b + 1]] = 1;
+    const int need = (int)std::count(bonded.begin() + std::min(L, n), bonded.end(), 1);
+    for (int P = (int)best.size() - 1; P >= 1 && P * (K - L) >= need; --P) {
         std::vector<std::vector<int>> got;
         for (int t = 0; t < SPIN_COVER_TRIES && got.empty(); ++t)
             got = spin_anneal_cover(n, sp, ibond, K, L, P, sp_mix(seed), SPIN_COVER_MOVES);
@@ -694,6 +896,14 @@ size_t spin_lds_bytes(int tsz, int ncls, int qq, bool cplx, int tpb)
     return std::max(t, sizeof(double) * 2 * (size_t)tpb);
 }
 
+// LDS bytes of one hv_spin_split block: tile, bond diagonals (at the end one sum per wave),
+// class coefficients
+size_t spin_split_lds(int tsz, int nbond, int ncls, int qq, bool cplx)
+{
+    return sizeof(double2) * ((size_t)tsz + (size_t)nbond * qq) +
+           std::max((size_t)ncls * qq * (cplx ? 16 : 8), (size_t)256);
+}
+
 struct SpinPlan {
     int K = 0, L = 0;
     std::vector<SpinPassDev> dev;
@@ -703,7 +913,9 @@ struct SpinPlan {
 };
 
 // Builds the passes for tile sites K (at most, fewer when the tables do not fit) and L forced
-// low sites (0: 3 if that costs no pass over 2, else 2).
+// low sites (0: 3 if that costs no pass over 2, else 2; where both vectors fit the 256 MB
+// Infinity Cache and short runs cost little, 1 if that saves a pass over 2, else 2: spin 1 on
+// 12 sites 2 passes for 3, 62 -> 56 us per H.v; on 16 sites, from HBM, 3 for 4 gain nothing).
 int spin_make_plan(int n, int q, int ibond, const std::vector<int32_t> &sp, const std::vector<int32_t> &btype,
                    const std::vector<double> &xl, const std::vector<int32_t> &ll, int Kmax, int Lreq, SpinPlan &plan)
 {
@@ -726,9 +938,19 @@ int spin_make_plan(int n, int q, int ibond, const std::vector<int32_t> &sp, cons
             cov = spin_cover(n, sp, ibond, K, L);
         } else {
             auto c2 = spin_cover(n, sp, ibond, K, std::min(2, K));
-            auto c3 = (K >= 3) ? spin_cover(n, sp, ibond, K, 3) : std::vector<std::vector<int>>{};
-            if (!c3.empty() && (c2.empty() || c3.size() <= c2.size())) { cov = c3; L = 3; }
-            else { cov = c2; L = std::min(2, K); }
+            if (32.0 * std::pow((double)q, (double)n) <= 256.0 * (1 << 20)) {
+                auto npass = [&](const std::vector<std::vector<int>> &c) {
+                    return spin_split(spin_balance(c, sp, n, ibond, w), btype, tcls).size();
+                };
+                auto c1 = spin_cover(n, sp, ibond, K, 1);
+                const bool one = !c1.empty() && (c2.empty() || npass(c1) < npass(c2));
+                cov = one ? c1 : c2;
+                L = one ? 1 : std::min(2, K);
+            } else {
+                auto c3 = (K >= 3) ? spin_cover(n, sp, ibond, K, 3) : std::vector<std::vector<int>>{};
+                if (!c3.empty() && (c2.empty() || c3.size() <= c2.size())) { cov = c3; L = 3; }
+                else { cov = c2; L = std::min(2, K); }
+            }
         }
         // tiles too small to hold every bond next to the forced sites: force fewer
         while (cov.empty() && L > 0) cov = spin_cover(n, sp, ibond, K, --L);
@@ -922,6 +1144,43 @@ static int launch_spin_pass(pned_ctx *ctx, int grid_cap, size_t lds, bool cplx, 
     return grid;
 }
 
+// The same pass by hv_spin_split, where R / S blocks to a tile are resident all at once
+// (S = 1 if that fits, else S = q): returns the grid, or 0 to leave it to hv_spin_pass.
+// Decided once per plan and pass (ctx->spin_split).
+template <int Q, int NR, int TPB>
+static int launch_spin_split(pned_ctx *ctx, int p, bool cplx, const pned_vec *v1, pned_vec *v0,
+                             const SpinPassDev *pd, const SpinPassArgs &a, double *part)
+{
+    constexpr int R = (NR == 2) ? Q * Q : Q;
+    using K = void (*)(const double2 *, double2 *, const SpinPassDev *, SpinPassArgs, double *);
+    const K k1 = cplx ? (K)hv_spin_split<Q, NR, TPB, 1, true> : (K)hv_spin_split<Q, NR, TPB, 1, false>;
+    K kq = nullptr;
+    if constexpr (R > Q) kq = cplx ? (K)hv_spin_split<Q, NR, TPB, Q, true> : (K)hv_spin_split<Q, NR, TPB, Q, false>;
+    const size_t lds = spin_split_lds(a.tsz, a.nbond, a.ncls, Q * Q, cplx);
+    int &parts = ctx->spin_split[p];
+    if (parts < 0) {
+        parts = 0;
+        if (ctx->num_cu <= 0 &&
+            hipDeviceGetAttribute(&ctx->num_cu, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess)
+            ctx->num_cu = 0;
+        for (const K k : {k1, kq}) {
+            int per_cu = 0;
+            const int np = (k == k1) ? R : R / Q;
+            if (!k || parts > 0 || lds > 160 * 1024) continue;
+            (void)hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k, TPB, lds) != hipSuccess)
+                per_cu = 0;
+            const uint64_t fit = std::min<uint64_t>((uint64_t)ctx->num_cu * (uint64_t)per_cu, SP_GRID_CAP);
+            if (a.tile_count * (uint64_t)np <= fit) parts = np;
+        }
+    }
+    if (parts == 0) return 0;
+    const int grid = (int)a.tile_count * parts;
+    hipLaunchKernelGGL(parts == R ? k1 : kq, dim3(grid), dim3(TPB), lds, ctx->stream, (const double2 *)v1->data,
+                       (double2 *)v0->data, pd, a, part);
+    return grid;
+}
+
 int launch_hv_spin_tiled(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double eperbd, bool fresh,
                          double *prdct_host, double xs, double ys)
 {
@@ -950,9 +1209,10 @@ int launch_hv_spin_tiled_shift(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, 
         ctx->spin_nlo = plan.nlo;
         ctx->spin_ncls = plan.ncls;
         ctx->spin_cplx = plan.cplx;
+        ctx->spin_split.assign(np, -1);
     }
     const int np = ctx->spin_np;
-    const int grid_cap = 2048;
+    const int grid_cap = SP_GRID_CAP;
     PNED_TRY(ensure_partial(ctx, 2 * (size_t)grid_cap * np + 16));
     PNED_TRY(ensure_result(ctx, 8));
     int rows = 0;
@@ -981,6 +1241,14 @@ int launch_hv_spin_tiled_shift(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, 
         const int R = (a.tsz + tpb - 1) / tpb;
         const bool cplx = ctx->spin_cplx[p] != 0;
         const size_t lds = spin_lds_bytes(a.tsz, a.ncls, qq, cplx, tpb);
+        // one thread per state of the tile's low digits, K - 2 (spin 1) or K - 1 of them
+        if (q == 3 && a.K == 8) grid = launch_spin_split<3, 2, 768>(ctx, p, cplx, v1, v0, pd, a, part);
+        else if (q == 3 && a.K >= 2) grid = launch_spin_split<3, 2, 256>(ctx, p, cplx, v1, v0, pd, a, part);
+        else if (q == 4 && a.K == 6) grid = launch_spin_split<4, 1, 1024>(ctx, p, cplx, v1, v0, pd, a, part);
+        else if (q == 4 && a.K >= 2) grid = launch_spin_split<4, 1, 256>(ctx, p, cplx, v1, v0, pd, a, part);
+        else if (q == 5 && a.K == 5) grid = launch_spin_split<5, 1, 640>(ctx, p, cplx, v1, v0, pd, a, part);
+        else if (q == 5 && a.K >= 2) grid = launch_spin_split<5, 1, 128>(ctx, p, cplx, v1, v0, pd, a, part);
+        if (grid == 0) {
 #define PNED_SPIN_CASE(QV, TV, RV)                                                                                   \
         if (q == QV && tpb == TV && R == RV) {                                                                      \
             grid = launch_spin_pass<QV, TV, RV>(ctx, grid_cap, lds, cplx, v1, v0, pd, a, part);                     \
@@ -991,6 +1259,7 @@ int launch_hv_spin_tiled_shift(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, 
         PNED_SPIN_CASE(5, 1024, 4) PNED_SPIN_CASE(5, 256, 3) PNED_SPIN_CASE(5, 256, 1)
         { return fail(PNED_E_UNSUPPORTED, "no tiled spin-S kernel instance for this q / tile"); }
 #undef PNED_SPIN_CASE
+        }
         PNED_HIP(hipGetLastError());
         rows += grid;
     }

@@ -259,6 +259,7 @@ struct pned_ctx {
     void *spin_pd = nullptr;         // tiled-pass tables
     int spin_K = -1, spin_np = 0;
     std::vector<int> spin_nb, spin_tsz, spin_nlo, spin_ncls, spin_cplx;
+    std::vector<int> spin_split;     // per pass: blocks per tile (hv_spin_split), 0 hv_spin_pass, -1 not decided
     // scratch for reductions: per-block partials and final results (pinned host mirror)
     double *d_partial = nullptr;
     size_t partial_cap = 0;          // in doubles

@@ -54,3 +54,25 @@ def test_split_matches_tiles(spec, cols, dtype):
         got.append(out)
     for p, q in zip(*got):
         assert np.array_equal(p, q)
+
+
+# hv_spin_split against the per-state gather kernel: one tile, several, parts of one and of q
+# slots, complex coefficients (field), tiles of few states, and tiles too many for it (hv_spin_pass)
+@pytest.mark.parametrize("spec,q,tile", [("2x2", 3, 0), ("2x2", 3, 6), ("2x3", 3, 0), ("2x3", 3, 7), ("2x3", 3, 4),
+                                         ("2x2", 4, 0), ("2x2", 4, 4), ("2x2", 5, 0), ("2x2", 5, 3)])
+@pytest.mark.parametrize("field", [0.0, 0.2])
+def test_spin_split_matches_gather(spec, q, tile, field):
+    ctx = gpu.Context(model.build_operator(lattice.get_cluster(spec), 20, 108.0, q=q, field=field))
+    if tile:
+        ctx.tune(tile_bits=tile)
+    x, a, b = (ctx.vector() for _ in range(3))
+    ctx.set_initial_vec(x, 5)
+    ctx.set_initial_vec(a, 6)
+    b.copy_from(a)
+    pa = ctx.p_mltply_v3(x, a, 0.03)
+    ctx.spin_kernel(False)
+    pb = ctx.p_mltply_v3(x, b, 0.03)
+    a, b = a.download(), b.download()
+    # at most 18 bonds of 9 elements a state, one rounding each: 162 * 1.1e-16, twice
+    assert np.linalg.norm(a - b) <= 1e-13 * np.linalg.norm(b)
+    assert abs(pa - pb) <= 1e-13 * np.linalg.norm(b)
