@@ -609,6 +609,12 @@ __global__ __launch_bounds__(RED_TPB) void k_tps_obs(const typename V2<Real>::T 
 // (phase A, spread over the block's threads), then every element of the chunk reads its
 // state's weights (phase B).  A thread's elements all lie in one column, so the block
 // reduction per column is the fixed tree of reduce_rows.
+//
+// Bound by the three vector reads: N=24 with 64 complex64 columns 9.28 -> 5.50 ms, 2.8 -> 4.7
+// TB/s.  B elements are loaded before the first is used (one at a time left too few loads in
+// flight; 6.67 ms), and the block sums use the weights' LDS, half of the outputs at a time, so
+// that four blocks of 128 VGPRs are resident on a CU and RED_GRID is one round of them.  Loading
+// the first batch ahead of phase A costs registers and with them a block: 6.35 ms.
 constexpr int TPS_CS_MAX = 256;   // states per chunk
 
 template <typename Real, int NOUT>
@@ -619,9 +625,11 @@ __global__ __launch_bounds__(RED_TPB) void k_tps_fused(const typename V2<Real>::
                                                        int cs, double *__restrict__ partial)
 {
     extern __shared__ double red[];
-    double *wt = red + NOUT * RED_TPB;   // [cs][1 + 2 nsq]: wzz, then (Re, Im) W_k
+    double *wt = red;   // [cs][1 + 2 nsq]: wzz, then (Re, Im) W_k; the block sums after the last chunk
     const ObsArgs &a = *ap;
     const int tid = threadIdx.x;
+    using V = typename V2<Real>::T;
+    constexpr int B = sizeof(Real) == 8 ? 2 : 4;   // elements in flight
     const int nsq = (10 + 2 * a.nsq <= NOUT) ? a.nsq : (NOUT - 10) / 2;
     const int nw = 1 + 2 * nsq;
     const int lc = __ffs(ncol) - 1;   // log2 ncol
@@ -650,49 +658,66 @@ __global__ __launch_bounds__(RED_TPB) void k_tps_fused(const typename V2<Real>::
         __syncthreads();
         // phase B: the chunk's elements
         const int nel = ns << lc;
-        for (int le = tid; le < nel; le += RED_TPB) {
-            const size_t e = (s0c << lc) + (size_t)le;
-            const double *ws = wt + (le >> lc) * nw;
-            double pr, pi, xr, xi, wr, wi;
-            ld(up, e, pr, pi);
-            ld(u, e, xr, xi);
-            ld(w, e, wr, wi);
-            acc[0] = fma(wr, wr, fma(wi, wi, acc[0]));
-            acc[2] = fma(pr, wr, fma(pi, wi, acc[2]));
-            acc[3] = fma(pr, wi, fma(-pi, wr, acc[3]));
-            acc[4] = fma(pr, xr, fma(pi, xi, acc[4]));
-            acc[5] = fma(pr, xi, fma(-pi, xr, acc[5]));
-            const double wzz = ws[0];
-            acc[6] = fma(wzz, xr * xr + xi * xi, acc[6]);
-            acc[8] = fma(wzz, pr * xr + pi * xi, acc[8]);
-            acc[9] = fma(wzz, pr * xi - pi * xr, acc[9]);
+        for (int le0 = tid; le0 < nel; le0 += B * RED_TPB) {
+            V pv[B], xv[B], wv[B];
 #pragma unroll
-            for (int k = 0; 10 + 2 * k + 1 < NOUT; ++k) {
-                if (k >= nsq) break;
-                const double cr = ws[1 + 2 * k], ci = ws[2 + 2 * k];
-                const double yr = cr * xr - ci * xi, yi = cr * xi + ci * xr;
-                double lr = xr, li = xi;
-                if (a.sq_left[k]) { lr = pr; li = pi; }
-                acc[10 + 2 * k] = fma(lr, yr, fma(li, yi, acc[10 + 2 * k]));
-                acc[10 + 2 * k + 1] = fma(lr, yi, fma(-li, yr, acc[10 + 2 * k + 1]));
+            for (int j = 0; j < B; ++j) {
+                const size_t e = (s0c << lc) + (size_t)min(le0 + j * RED_TPB, nel - 1);
+                pv[j] = up[e];
+                xv[j] = u[e];
+                wv[j] = w[e];
+            }
+#pragma unroll
+            for (int j = 0; j < B; ++j) {
+                const int le = le0 + j * RED_TPB;
+                if (le >= nel) break;
+                const double *ws = wt + (le >> lc) * nw;
+                const double pr = (double)pv[j].x, pi = (double)pv[j].y, xr = (double)xv[j].x, xi = (double)xv[j].y;
+                const double wr = (double)wv[j].x, wi = (double)wv[j].y;
+                acc[0] = fma(wr, wr, fma(wi, wi, acc[0]));
+                acc[2] = fma(pr, wr, fma(pi, wi, acc[2]));
+                acc[3] = fma(pr, wi, fma(-pi, wr, acc[3]));
+                acc[4] = fma(pr, xr, fma(pi, xi, acc[4]));
+                acc[5] = fma(pr, xi, fma(-pi, xr, acc[5]));
+                const double wzz = ws[0];
+                acc[6] = fma(wzz, xr * xr + xi * xi, acc[6]);
+                acc[8] = fma(wzz, pr * xr + pi * xi, acc[8]);
+                acc[9] = fma(wzz, pr * xi - pi * xr, acc[9]);
+#pragma unroll
+                for (int k = 0; 10 + 2 * k + 1 < NOUT; ++k) {
+                    if (k >= nsq) break;
+                    const double cr = ws[1 + 2 * k], ci = ws[2 + 2 * k];
+                    const double yr = cr * xr - ci * xi, yi = cr * xi + ci * xr;
+                    double lr = xr, li = xi;
+                    if (a.sq_left[k]) { lr = pr; li = pi; }
+                    acc[10 + 2 * k] = fma(lr, yr, fma(li, yi, acc[10 + 2 * k]));
+                    acc[10 + 2 * k + 1] = fma(lr, yi, fma(-li, yr, acc[10 + 2 * k + 1]));
+                }
             }
         }
         __syncthreads();
     }
+    // the block sums per column, half of the outputs at a time
+    constexpr int NH = NOUT / 2;
+    static_assert(NOUT % 2 == 0, "outputs in two halves");
 #pragma unroll
-    for (int k = 0; k < NOUT; ++k) red[NOUT * tid + k] = acc[k];
-    __syncthreads();
-    for (int s2 = RED_TPB / 2; s2 >= ncol && s2 > 0; s2 >>= 1) {
-        if (tid < s2) {
+    for (int h = 0; h < NOUT; h += NH) {
+        if (h > 0) __syncthreads();
 #pragma unroll
-            for (int k = 0; k < NOUT; ++k) red[NOUT * tid + k] += red[NOUT * (tid + s2) + k];
-        }
+        for (int k = 0; k < NH; ++k) red[NH * tid + k] = acc[h + k];
         __syncthreads();
-    }
-    if (tid < ncol) {
+        for (int s2 = RED_TPB / 2; s2 >= ncol && s2 > 0; s2 >>= 1) {
+            if (tid < s2) {
 #pragma unroll
-        for (int k = 0; k < NOUT; ++k)
-            partial[(size_t)blockIdx.x * NOUT * ncol + NOUT * tid + k] = red[NOUT * tid + k];
+                for (int k = 0; k < NH; ++k) red[NH * tid + k] += red[NH * (tid + s2) + k];
+            }
+            __syncthreads();
+        }
+        if (tid < ncol) {
+#pragma unroll
+            for (int k = 0; k < NH; ++k)
+                partial[(size_t)blockIdx.x * NOUT * ncol + NOUT * tid + h + k] = red[NH * tid + k];
+        }
     }
 }
 
@@ -1446,7 +1471,7 @@ static int tps_reduce_shape(const pned_vec *u, int nsq, TpsReduceShape &s)
     s.cs = std::max(1, std::min(TPS_CS_MAX, 64 * RED_TPB / u->nvec));
     const size_t nchunk = ((size_t)u->dim + s.cs - 1) / s.cs;
     s.grid = (int)std::min<size_t>(nchunk, (size_t)RED_GRID);
-    s.lds = sizeof(double) * ((size_t)TPS_RED_WIDTH * RED_TPB + (size_t)s.cs * (1 + 2 * nsq));
+    s.lds = sizeof(double) * std::max((size_t)TPS_RED_WIDTH / 2 * RED_TPB, (size_t)s.cs * (1 + 2 * nsq));
     return PNED_OK;
 }
 
