@@ -298,9 +298,9 @@ int cocg_update(pned_ctx *ctx, const pned_vec *p, const pned_vec *y, pned_vec *x
 // after such steps: v1 <- sx x, v0 <- y + a sx x, (x, y) = (v1, v0) or, swapped, (v0, v1)
 int lanczos_lazy_restore(pned_ctx *ctx, pned_vec *v1, pned_vec *v0, bool swapped, double sx, double a);
 // lanczos_lazy_step's enqueue-only form (one column, S=1/2 full space), which Lanczos
-// loops capture into graphs: st = [sx, sy, prd re, prd im, b2 of the step before] on the
-// device; the step sets sx = 1/sqrt(b2), sy = -sqrt(b2) sx (fresh: 1, 0), runs the step and
-// writes [prd re, prd im, b2] to slot and b2 to st[4].  No allocation or host wait once
+// loops capture into graphs: st = [sx, sy] on the device (fresh: set to 1, 0); the step runs
+// with them, writes [prd re, prd im, b2] to slot and sets sx = 1/sqrt(b2), sy = -sqrt(b2) sx
+// for the next.  No allocation or host wait once
 // lanczos_lazy_setup (which also checks the pair) and one un-captured step of the same
 // shape have run.
 int lanczos_lazy_setup(pned_ctx *ctx, const pned_vec *x, const pned_vec *y);
@@ -385,12 +385,12 @@ int tps_fused_reduce(pned_ctx *ctx, const pned_vec *up, const pned_vec *u, const
 constexpr int TPS_RED_WIDTH = 26;
 // the captured form of the fused mTPQ step: a device copy of the observable tables
 // (*dobs, freed by the caller with hipFree), then per step, enqueued only (no allocation, no
-// host round trip): su = 1/sqrt(red_prev[c][0]) (1 when red_prev is null), w = (L-H)(su u),
-// slot[0..2nc) = the H.v's per-column product (what pned_tps_fused reads back),
-// slot[2nc..) = the reduction of (up, u, w) ([column][TPS_RED_WIDTH])
+// host round trip): w = (L-H)(su u) (first: su = 1), slot[0..2nc) = the H.v's per-column
+// product (what pned_tps_fused reads back), slot[2nc..) = the reduction of (up, u, w)
+// ([column][TPS_RED_WIDTH]), su = 1/sqrt(|w|^2) for the next step
 int tps_graph_setup(pned_ctx *ctx, const pned_vec *u, void **dobs, int *nsq);
 int tps_graph_step(pned_ctx *ctx, const pned_vec *up, const pned_vec *u, pned_vec *w, const void *dobs, int nsq,
-                   const double *red_prev, double *su_dev, double *slot);
+                   bool first, double *su_dev, double *slot);
 int renbun_gpu(pned_ctx *ctx, int i_range, int s_maxitr, double split, double ene, double eta,
                const double *salpha, const double *sbeta, double *w, double *dsf, int *conv);
 

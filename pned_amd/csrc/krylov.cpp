@@ -38,7 +38,7 @@ struct LanczosSteps {
     bool lazy, dev;
     pned_vec *X, *Y;
     double sx = 1.0, sy = 0.0;
-    double *st = nullptr;     // device: [sx, sy, prd re, prd im, beta^2], then GRAPH_STEPS slots of 3
+    double *st = nullptr;     // device: [sx, sy], then GRAPH_STEPS slots of [prd re, prd im, beta^2]
     double *host = nullptr;   // pinned read-back of the slots
     hipGraph_t graph[2] = {nullptr, nullptr};
     hipGraphExec_t exec[2] = {nullptr, nullptr};
@@ -83,7 +83,7 @@ struct LanczosSteps {
     // first step of a run); b1 carries the beta before them
     int harvest(int n, bool fresh, double &b1, double *a_out, double *b_out)
     {
-        PNED_HIP(hipMemcpyAsync(host, st + 5, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, ctx->stream));
+        PNED_HIP(hipMemcpyAsync(host, st + 2, sizeof(double) * 3 * n, hipMemcpyDeviceToHost, ctx->stream));
         PNED_HIP(hipStreamSynchronize(ctx->stream));
         for (int j = 0; j < n; ++j) {
             if (!(fresh && j == 0)) roll(b1);
@@ -98,9 +98,9 @@ struct LanczosSteps {
     {
         if (dev) {
             PNED_TRY(lanczos_lazy_setup(ctx, X, Y));
-            PNED_HIP(hipMalloc((void **)&st, sizeof(double) * (5 + 3 * GRAPH_STEPS)));
+            PNED_HIP(hipMalloc((void **)&st, sizeof(double) * (2 + 3 * GRAPH_STEPS)));
             PNED_HIP(hipHostMalloc((void **)&host, sizeof(double) * 3 * GRAPH_STEPS, hipHostMallocDefault));
-            PNED_TRY(lanczos_lazy_enqueue(ctx, X, Y, true, st, st + 5));
+            PNED_TRY(lanczos_lazy_enqueue(ctx, X, Y, true, st, st + 2));
             return harvest(1, true, b1, &a1, &b1);
         }
         if (lazy) return lazy_ab(true, a1, b1);
@@ -112,7 +112,7 @@ struct LanczosSteps {
     {
         if (dev) {
             // enqueued with the roles after the swap that harvest's roll() mirrors
-            PNED_TRY(lanczos_lazy_enqueue(ctx, Y, X, false, st, st + 5));
+            PNED_TRY(lanczos_lazy_enqueue(ctx, Y, X, false, st, st + 2));
             return harvest(1, false, b1, &a1, &b1);
         }
         if (lazy) {
@@ -131,7 +131,7 @@ struct LanczosSteps {
         int rc = PNED_OK;
         for (int j = 0; j < GRAPH_STEPS && rc == PNED_OK; ++j) {
             std::swap(x, y);
-            rc = lanczos_lazy_enqueue(ctx, x, y, false, st, st + 5 + 3 * j);
+            rc = lanczos_lazy_enqueue(ctx, x, y, false, st, st + 2 + 3 * j);
         }
         const hipError_t ec = hipStreamEndCapture(ctx->stream, &graph[role]);
         PNED_TRY(rc);
@@ -931,12 +931,11 @@ int pned_tps_fused_graph(pned_ctx *ctx, pned_vec *v1, pned_vec *va, pned_vec *vb
     pned_vec *u = v1, *up = va, *w = vb;
     PNED_TRY(pned_vec_zero(ctx, up));
     std::vector<double> su(nc, 1.0), sp(nc, 0.0);
-    // step i (1-based) writes slot (i - 2) mod G and scales by the slot before it
+    // step i (1-based) writes slot (i - 2) mod G
     auto slot_of = [G](int i) { return ((i - 2) % G + G) % G; };
     auto enqueue = [&](int i) -> int {
         const int sl = slot_of(i);
-        const double *prev = i == 1 ? nullptr : run.hist + (size_t)slot_of(i - 1) * slot_d + 2 * (size_t)nc;
-        PNED_TRY(tps_graph_step(ctx, up, u, w, run.dobs, nsq, prev, run.su, run.hist + (size_t)sl * slot_d));
+        PNED_TRY(tps_graph_step(ctx, up, u, w, run.dobs, nsq, i == 1, run.su, run.hist + (size_t)sl * slot_d));
         pned_vec *t = up;   // vg <- v1, v1 <- v0, v0 <- free
         up = u;
         u = w;

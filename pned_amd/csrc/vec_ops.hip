@@ -957,38 +957,41 @@ int lanczos_lazy_step(pned_ctx *ctx, pned_vec *x, pned_vec *y, const double *sx,
     return PNED_OK;
 }
 
-__global__ void k_copy_f64(const double *__restrict__ src, double *__restrict__ dst, int n)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = src[i];
-}
-
-// the captured form's scalars: st = [sx, sy, prd re, prd im, b2 of the step before]
-__global__ void k_lz_scale(double *__restrict__ st, int fresh)
+// the captured form's scalars: st = [sx, sy] of the step to come (1, 0 for the first)
+__global__ void k_lz_start(double *__restrict__ st)
 {
     if (threadIdx.x != 0) return;
-    if (fresh) {
-        st[0] = 1.0;
-        st[1] = 0.0;
-    } else {
-        const double b = sqrt(st[4]), sxo = st[0];   // v1 is y / b, v0 is x times -b sx
-        st[0] = 1.0 / b;
-        st[1] = -b * sxo;
+    st[0] = 1.0;
+    st[1] = 0.0;
+}
+
+// End of a captured step in one launch of one block (three launches of 4 us each before it):
+// beta^2 from the partials of k_lanczos_lazy, summed as reduce_rows does (nrows > 0), or from
+// the H.v's result ([prd re, prd im, b2], nrows = 0); slot = [prd re, prd im, b2]; st = the
+// scales of the next step.
+__global__ __launch_bounds__(256) void k_lz_end(const double *__restrict__ result, const double *__restrict__ partial,
+                                                int nrows, double *__restrict__ st, double *__restrict__ slot)
+{
+    __shared__ double red[256];
+    const int tid = threadIdx.x;
+    if (nrows > 0) {
+        double s = 0.0;
+        for (int b = tid; b < nrows; b += 256) s += partial[b];
+        red[tid] = s;
+        __syncthreads();
+        for (int k = 128; k > 0; k >>= 1) {
+            if (tid < k) red[tid] += red[tid + k];
+            __syncthreads();
+        }
     }
-}
-
-// slot = [prd re, prd im, b2], st[4] = b2; fused: all three from the H.v's result
-// ([prd re, prd im, b2]), else prd from st[2..4) and b2 from the beta kernel's result
-__global__ void k_lz_store(const double *__restrict__ result, double *__restrict__ st, double *__restrict__ slot,
-                           int fused)
-{
-    if (threadIdx.x != 0) return;
-    const double pr = fused ? result[0] : st[2], pi = fused ? result[1] : st[3];
-    const double b2 = fused ? result[2] : result[0];
-    slot[0] = pr;
-    slot[1] = pi;
+    if (tid != 0) return;
+    const double b2 = nrows > 0 ? red[0] : result[2];
+    slot[0] = result[0];
+    slot[1] = result[1];
     slot[2] = b2;
-    st[4] = b2;
+    const double b = sqrt(b2), sxo = st[0];   // v1 is y / b, v0 is x times -b sx
+    st[0] = 1.0 / b;
+    st[1] = -b * sxo;
 }
 
 int lanczos_lazy_setup(pned_ctx *ctx, const pned_vec *x, const pned_vec *y)
@@ -1003,8 +1006,10 @@ int lanczos_lazy_enqueue(pned_ctx *ctx, pned_vec *x, pned_vec *y, bool fresh, do
     PNED_TRY(check_hv_pair(ctx, x, y));
     if (x->nvec != 1 || ctx->q != 2)
         return fail(PNED_E_UNSUPPORTED, "captured Lanczos step: one column of an S=1/2 context");
-    hipLaunchKernelGGL(k_lz_scale, dim3(1), dim3(64), 0, ctx->stream, st, fresh ? 1 : 0);
-    PNED_HIP(hipGetLastError());
+    if (fresh) {
+        hipLaunchKernelGGL(k_lz_start, dim3(1), dim3(64), 0, ctx->stream, st);
+        PNED_HIP(hipGetLastError());
+    }
     bool fused = false;
     if (ctx->sector_k >= 0)
         PNED_TRY(launch_hv_sector(ctx, x, y, 0.0, fresh, nullptr, st, fresh ? nullptr : st + 1));
@@ -1012,22 +1017,18 @@ int lanczos_lazy_enqueue(pned_ctx *ctx, pned_vec *x, pned_vec *y, bool fresh, do
         PNED_TRY(launch_hv_s12(ctx, x, y, 0.0, fresh, nullptr, st, fresh ? nullptr : st + 1, &fused));
     if (!fused) {
         const size_t nelem = (size_t)x->dim;
-        hipLaunchKernelGGL(k_copy_f64, dim3(1), dim3(64), 0, ctx->stream, ctx->d_result, st + 2, 2);
-        PNED_HIP(hipGetLastError());
         if (x->dtype == PNED_C128)
             hipLaunchKernelGGL(k_lanczos_lazy<double>, dim3(RED_GRID), dim3(RED_TPB), 0, ctx->stream,
                                (const double2 *)x->data, (double2 *)y->data, (const double *)st,
-                               (const double *)(st + 2), nelem, 1, ctx->d_partial);
+                               (const double *)ctx->d_result, nelem, 1, ctx->d_partial);
         else
             hipLaunchKernelGGL(k_lanczos_lazy<float>, dim3(RED_GRID), dim3(RED_TPB), 0, ctx->stream,
                                (const float2 *)x->data, (float2 *)y->data, (const double *)st,
-                               (const double *)(st + 2), nelem, 1, ctx->d_partial);
-        PNED_HIP(hipGetLastError());
-        hipLaunchKernelGGL(reduce_rows, dim3(1), dim3(256), 0, ctx->stream, ctx->d_partial, RED_GRID, 1,
-                           ctx->d_result);
+                               (const double *)ctx->d_result, nelem, 1, ctx->d_partial);
         PNED_HIP(hipGetLastError());
     }
-    hipLaunchKernelGGL(k_lz_store, dim3(1), dim3(64), 0, ctx->stream, ctx->d_result, st, slot, fused ? 1 : 0);
+    hipLaunchKernelGGL(k_lz_end, dim3(1), dim3(256), 0, ctx->stream, ctx->d_result, ctx->d_partial,
+                       fused ? 0 : RED_GRID, st, slot);
     PNED_HIP(hipGetLastError());
     return PNED_OK;
 }
@@ -1475,13 +1476,12 @@ static int tps_reduce_shape(const pned_vec *u, int nsq, TpsReduceShape &s)
     return PNED_OK;
 }
 
-// k_tps_fused over (up, u, w) into ctx->d_partial, then the final reduction into out_dev
-// ([column][TPS_RED_WIDTH]); dargs is a device copy of the context's ObsArgs.  Enqueued
-// only: no allocation, no host round trip (the partial buffer must already hold the grid)
-static int tps_fused_reduce_launch(pned_ctx *ctx, const pned_vec *up, const pned_vec *u, const pned_vec *w,
-                                   const ObsArgs *dargs, int nsq, double *out_dev)
+// k_tps_fused over (up, u, w) into s.grid rows of ctx->d_partial; dargs is a device copy of the
+// context's ObsArgs.  Enqueued only: no allocation, no host round trip (the partial buffer must
+// already hold the grid)
+static int tps_fused_launch(pned_ctx *ctx, const pned_vec *up, const pned_vec *u, const pned_vec *w,
+                            const ObsArgs *dargs, int nsq, TpsReduceShape &s)
 {
-    TpsReduceShape s;
     PNED_TRY(tps_reduce_shape(u, nsq, s));
     const size_t nstates = (size_t)u->dim;
     if (u->dtype == PNED_C128) {
@@ -1497,9 +1497,6 @@ static int tps_fused_reduce_launch(pned_ctx *ctx, const pned_vec *up, const pned
                            (const float2 *)u->data, (const float2 *)w->data, dargs, nstates, u->nvec, s.cs,
                            ctx->d_partial);
     }
-    PNED_HIP(hipGetLastError());
-    hipLaunchKernelGGL(reduce_rows, dim3(TPS_RED_WIDTH * u->nvec), dim3(256), 0, ctx->stream, ctx->d_partial, s.grid,
-                       TPS_RED_WIDTH * u->nvec, out_dev);
     PNED_HIP(hipGetLastError());
     return PNED_OK;
 }
@@ -1522,7 +1519,10 @@ int tps_fused_reduce(pned_ctx *ctx, const pned_vec *up, const pned_vec *u, const
     std::vector<double> hbuf(nd);
     std::memcpy(hbuf.data(), &a, sizeof(ObsArgs));
     PNED_TRY(upload_scalars(ctx, hbuf.data(), nd, &dargs));
-    PNED_TRY(tps_fused_reduce_launch(ctx, up, u, w, (const ObsArgs *)dargs, nsq, ctx->d_result));
+    PNED_TRY(tps_fused_launch(ctx, up, u, w, (const ObsArgs *)dargs, nsq, s));
+    hipLaunchKernelGGL(reduce_rows, dim3(TPS_RED_WIDTH * u->nvec), dim3(256), 0, ctx->stream, ctx->d_partial, s.grid,
+                       TPS_RED_WIDTH * u->nvec, ctx->d_result);
+    PNED_HIP(hipGetLastError());
     const size_t all = (size_t)TPS_RED_WIDTH * u->nvec;
     PNED_HIP(hipMemcpyAsync(ctx->h_result, ctx->d_result, sizeof(double) * all, hipMemcpyDeviceToHost, ctx->stream));
     PNED_HIP(hipStreamSynchronize(ctx->stream));
@@ -1531,11 +1531,35 @@ int tps_fused_reduce(pned_ctx *ctx, const pned_vec *up, const pned_vec *u, const
     return PNED_OK;
 }
 
-// su[c] = 1 / sqrt(red[c][0]) (1/||v0|| of the previous step), or 1 without a previous step
-__global__ void k_tps_scale(const double *__restrict__ red, int nc, double *__restrict__ su)
+// su[c] = 1 for the first step
+__global__ void k_tps_start(int nc, double *__restrict__ su)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < nc) su[c] = red ? 1.0 / sqrt(red[(size_t)c * TPS_RED_WIDTH]) : 1.0;
+    if (c < nc) su[c] = 1.0;
+}
+
+// End of a captured step: the final sums of k_tps_fused as reduce_rows forms them, and with
+// them (two launches of 4 us each before) the H.v's 2 nc sums into slot and the next step's
+// scale su[c] = 1 / sqrt(|w|^2) from the block that sums it.  slot = [2 nc | nc TPS_RED_WIDTH].
+__global__ __launch_bounds__(256) void k_tps_end(const double *__restrict__ partial, int nrows, int nc,
+                                                 const double *__restrict__ prd, double *__restrict__ slot,
+                                                 double *__restrict__ su)
+{
+    __shared__ double red[256];
+    const int c = blockIdx.x, tid = threadIdx.x, width = TPS_RED_WIDTH * nc;
+    if (tid == 0 && c < 2 * nc) slot[c] = prd[c];
+    double s = 0.0;
+    for (int b = tid; b < nrows; b += 256) s += partial[(size_t)b * width + c];
+    red[tid] = s;
+    __syncthreads();
+    for (int k = 128; k > 0; k >>= 1) {
+        if (tid < k) red[tid] += red[tid + k];
+        __syncthreads();
+    }
+    if (tid == 0) {
+        slot[2 * nc + c] = red[0];
+        if (c % TPS_RED_WIDTH == 0) su[c / TPS_RED_WIDTH] = 1.0 / sqrt(red[0]);
+    }
 }
 
 int tps_graph_setup(pned_ctx *ctx, const pned_vec *u, void **dobs, int *nsq)
@@ -1559,17 +1583,22 @@ int tps_graph_setup(pned_ctx *ctx, const pned_vec *u, void **dobs, int *nsq)
 }
 
 int tps_graph_step(pned_ctx *ctx, const pned_vec *up, const pned_vec *u, pned_vec *w, const void *dobs, int nsq,
-                   const double *red_prev, double *su_dev, double *slot)
+                   bool first, double *su_dev, double *slot)
 {
     PNED_TRY(check_hv_pair(ctx, u, w));
     PNED_TRY(check_hv_pair(ctx, up, u));
     const int nc = u->nvec;
-    hipLaunchKernelGGL(k_tps_scale, dim3((nc + 63) / 64), dim3(64), 0, ctx->stream, red_prev, nc, su_dev);
-    PNED_HIP(hipGetLastError());
+    if (first) {
+        hipLaunchKernelGGL(k_tps_start, dim3((nc + 63) / 64), dim3(64), 0, ctx->stream, nc, su_dev);
+        PNED_HIP(hipGetLastError());
+    }
     PNED_TRY(launch_hv_s12(ctx, u, w, 0.0, true, nullptr, su_dev));   // w = (L-H)(su u)
-    hipLaunchKernelGGL(k_copy_f64, dim3((2 * nc + 63) / 64), dim3(64), 0, ctx->stream, ctx->d_result, slot, 2 * nc);
+    TpsReduceShape s;
+    PNED_TRY(tps_fused_launch(ctx, up, u, w, (const ObsArgs *)dobs, nsq, s));
+    hipLaunchKernelGGL(k_tps_end, dim3(TPS_RED_WIDTH * nc), dim3(256), 0, ctx->stream, ctx->d_partial, s.grid, nc,
+                       ctx->d_result, slot, su_dev);
     PNED_HIP(hipGetLastError());
-    return tps_fused_reduce_launch(ctx, up, u, w, (const ObsArgs *)dobs, nsq, slot + 2 * nc);
+    return PNED_OK;
 }
 
 int renbun_gpu(pned_ctx *ctx, int i_range, int s_maxitr, double split, double ene, double eta,
