@@ -1202,16 +1202,21 @@ static int contiguous_bits(const std::vector<int> &b)
 
 // Threads of the untuned term-major plan, by its tile size (complex128 figures: one column with
 // field, us per H.v).  2^12-state tiles 1024 threads up to 2^21 elements (N=20 57.9, on 512 68), 512
-// above (N=24 533 against 565: two blocks per CU), but 1024 in batches (N=20 with 8 columns 277
-// against 344).  2^13 1024 (N=28 9.08 ms, on 512 13.9).  complex64: 2^12 512 (N=24 383, on 1024 472),
-// 2^13 1024 (N=28 5.8 ms), 2^14 512 (1024 spill; N=24 with 64 columns 28.7 against 31.7 ms).
+// above (N=24 533 against 565: two blocks per CU), but 1024 with columns of one operator (N=20 with
+// 8 columns 277 against 344); one operator per column 512 above as well (5 batch steps, N=20 with 8
+// columns 2.41 ms against 2.52).  2^11-state tiles 512: 4 slots a thread, 105 VGPRs against 169 on
+// 256 threads (5 batch steps, N=16 with 8 columns 464 us against 528, N=18 with 2 446 against 497;
+// 1024 threads 1000 against 897 at N=18 with 8).  2^13 1024 (N=28 9.08 ms, on 512 13.9).  complex64:
+// 2^12 512 (N=24 383, on 1024 472), 2^13 1024 (N=28 5.8 ms), 2^14 512 (1024 spill; N=24 with 64 columns
+// 28.7 against 31.7 ms).
 static int default_threads(const pned_ctx *ctx, const S12Plan &pl, int colbits, bool c128)
 {
     const int K = pl.passes.empty() ? 12 : pl.passes[0].K;
     const bool big = (double)ctx->dim * (double)(1ull << colbits) > (double)(1ull << 21);
-    if (K <= 11) return 256;
+    if (K <= 10) return 256;
+    if (K == 11) return 512;
     if (!c128) return K == 13 ? 1024 : 512;
-    return K == 12 && big && colbits == 0 ? 512 : 1024;
+    return K == 12 && big && (colbits == 0 || pl.nop > 1) ? 512 : 1024;
 }
 
 // the thread count whose register slots order a pass's terms (see build_tm_terms)

@@ -76,3 +76,24 @@ def test_spin_split_matches_gather(spec, q, tile, field):
     # at most 18 bonds of 9 elements a state, one rounding each: 162 * 1.1e-16, twice
     assert np.linalg.norm(a - b) <= 1e-13 * np.linalg.norm(b)
     assert abs(pa - pb) <= 1e-13 * np.linalg.norm(b)
+
+
+# one operator per column: the untuned plan (512 threads on 2^11-state tiles, and on 2^12-state tiles above
+# 2^21 elements) against 256 threads on the same plan rules
+@pytest.mark.parametrize("spec,cols", [("2x4", 8), (18, 2), ("2x5", 4)])
+def test_batch_threads(spec, cols):
+    cl = lattice.get_cluster(spec)
+    ops = [model.build_operator(cl, 20, 126.0 + 23.0 * c, field=0.1 + 0.01 * c) for c in range(cols)]
+    got = []
+    for threads in (0, 256):
+        ctx = gpu.Context(ops[0], batch_ops=ops)
+        if threads:
+            ctx.tune(0, 0, threads)
+        x, y = ctx.vector(cols), ctx.vector(cols)
+        ctx.set_initial_vec(x, 5)
+        a, b = ctx.lanczos_batch_steps(x, y, np.ones(cols, dtype=np.int32), np.zeros(cols), np.zeros(cols), 5)
+        got.append((a, b, x.download(), y.download()))
+    # the sums over 2^16 and more products differ in order: sqrt of their number times 1.1e-16, and five
+    # steps that each divide by a beta of order one
+    for p, q in zip(*got):
+        assert np.linalg.norm(p - q) <= 1e-12 * np.linalg.norm(q)
