@@ -295,6 +295,14 @@ int lanczos_lazy_step(pned_ctx *ctx, pned_vec *x, pned_vec *y, const double *sx,
 // COCG: x += a p, r -= a y; out4 = <r|r> (re, im), r^T r (re, im) of the new r
 int cocg_update(pned_ctx *ctx, const pned_vec *p, const pned_vec *y, pned_vec *x, pned_vec *r, const double *a,
                 double *out4);
+// the same with the scalars on the device (complex128): st = [rho, beta] (cocg_start checks the
+// shapes and sets rho); a step takes mu = p^T y from d_result, updates x, r, st and reads <r|r>
+// back into rr; cocg_direction forms p = r + beta p.  Nothing else may use the scalar upload
+// buffer, which holds st, between start and the last step
+int cocg_start(pned_ctx *ctx, const pned_vec *p, const pned_vec *y, const pned_vec *x, const pned_vec *r,
+               const double *rho, double **st);
+int cocg_direction(pned_ctx *ctx, const pned_vec *r, pned_vec *p, const double *st);
+int cocg_step(pned_ctx *ctx, const pned_vec *p, const pned_vec *y, pned_vec *x, pned_vec *r, double *st, double *rr);
 // after such steps: v1 <- sx x, v0 <- y + a sx x, (x, y) = (v1, v0) or, swapped, (v0, v1)
 int lanczos_lazy_restore(pned_ctx *ctx, pned_vec *v1, pned_vec *v0, bool swapped, double sx, double a);
 // lanczos_lazy_step's enqueue-only form (one column, S=1/2 full space), which Lanczos

@@ -605,16 +605,29 @@ int pned_cocg(pned_ctx *ctx, double e0, double eta, const pned_vec *b, pned_vec 
     const bool fused = ctx->q >= 3 && ctx->q <= 5 && ctx->spin_tiled && ctx->sector_k < 0 && p->ctx == ctx &&
                        y->ctx == ctx && p != y && p->nvec == 1 && y->nvec == 1 && p->dtype == PNED_C128 &&
                        y->dtype == PNED_C128 && p->dim == ctx->dim && y->dim == ctx->dim;
+    if (fused) {
+        // rho, mu and beta stay on the device: one wait per iteration, for the residual
+        double *st;
+        PNED_TRY(cocg_start(ctx, p, y, x, r, rho, &st));
+        for (int it = 1; it <= max_it; ++it) {
+            double rr;
+            if (it > 1) PNED_TRY(cocg_direction(ctx, r, p, st));   // p = r + beta p
+            // y = (H - e0 + i eta) p, mu = p^T y
+            PNED_TRY(launch_hv_spin_tiled_shift(ctx, p, y, eperbd, true, nullptr, 1.0, 1.0, 0.0, eta, true));
+            PNED_TRY(cocg_step(ctx, p, y, x, r, st, &rr));
+            *resid = std::sqrt(rr) / bnorm;
+            *iters = it;
+            if (*resid < tol) return PNED_OK;
+        }
+        PNED_TRY(cocg_direction(ctx, r, p, st));
+        PNED_HIP(hipStreamSynchronize(ctx->stream));
+        return fail(PNED_E_NOCONV, "cocg did not reach the tolerance");
+    }
     for (int it = 1; it <= max_it; ++it) {
         double pr[2], mu[2], rho2[2], rr[2];
-        if (fused) {
-            // y = (H - e0 + i eta) p, mu = p^T y
-            PNED_TRY(launch_hv_spin_tiled_shift(ctx, p, y, eperbd, true, mu, 1.0, 1.0, 0.0, eta, true));
-        } else {
-            PNED_TRY(pned_hv_fresh(ctx, p, y, eperbd, pr));      // y = (H - e0) p
-            PNED_TRY(pned_axpby(ctx, ieta, p, one, y));          // y += i eta p
-            PNED_TRY(dotu(ctx, p, y, mu));
-        }
+        PNED_TRY(pned_hv_fresh(ctx, p, y, eperbd, pr));      // y = (H - e0) p
+        PNED_TRY(pned_axpby(ctx, ieta, p, one, y));          // y += i eta p
+        PNED_TRY(dotu(ctx, p, y, mu));
         const std::complex<double> al = std::complex<double>(rho[0], rho[1]) / std::complex<double>(mu[0], mu[1]);
         const double pa[2] = {al.real(), al.imag()};
         double sums[4];

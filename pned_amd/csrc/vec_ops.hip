@@ -195,6 +195,18 @@ __global__ void k_lanczos_restore(typename V2<Real>::T *__restrict__ p1, typenam
     }
 }
 
+// a / b, the divisor scaled by a power of two so that |b|^2 neither overflows nor underflows
+__device__ __forceinline__ void cdiv(double ar, double ai, double br, double bi, double &qr, double &qi)
+{
+    const double m = fmax(fabs(br), fabs(bi));
+    const int e = (m > 0.0 && isfinite(m)) ? -ilogb(m) : 0;
+    br = ldexp(br, e);
+    bi = ldexp(bi, e);
+    const double d = br * br + bi * bi;
+    qr = ldexp((ar * br + ai * bi) / d, e);
+    qi = ldexp((ai * br - ar * bi) / d, e);
+}
+
 // one COCG update (one column): x += a p, r -= a y, and of the new r the sums
 // <r|r> (re, im) and r^T r (re, im): one pass over p, y, x, r instead of two axpy passes
 // and two reductions
@@ -203,9 +215,11 @@ __global__ __launch_bounds__(RED_TPB) void k_cocg_update(const typename V2<Real>
                                                          const typename V2<Real>::T *__restrict__ y,
                                                          typename V2<Real>::T *__restrict__ x,
                                                          typename V2<Real>::T *__restrict__ r, double ar, double ai,
-                                                         size_t nelem, double *__restrict__ partial)
+                                                         const double *__restrict__ rho,
+                                                         const double *__restrict__ mu, size_t nelem, double *__restrict__ partial)
 {
     __shared__ double red[4 * RED_TPB];
+    if (rho) cdiv(rho[0], rho[1], mu[0], mu[1], ar, ai);   // the scalars on the device
     const size_t stride = (size_t)RED_TPB * gridDim.x;
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
     for (size_t e = (size_t)blockIdx.x * RED_TPB + threadIdx.x; e < nelem; e += stride) {
@@ -224,6 +238,41 @@ __global__ __launch_bounds__(RED_TPB) void k_cocg_update(const typename V2<Real>
         acc[3] = fma(rr, ri, fma(ri, rr, acc[3]));
     }
     block_reduce_cols<4>(red, acc, 1, partial + (size_t)blockIdx.x * 4);
+}
+
+// the sums of k_cocg_update's partials (four groups of 256 threads, each as reduce_rows adds
+// them) into out[0..4), and from st = [rho, beta]: beta = r^T r / rho, rho = r^T r
+__global__ __launch_bounds__(1024) void k_cocg_end(const double *__restrict__ partial, int nrows,
+                                                   double *__restrict__ out, double *__restrict__ st)
+{
+    __shared__ double red[1024];
+    const int q = threadIdx.x >> 8, tid = threadIdx.x & 255;
+    double s = 0.0;
+    for (int b = tid; b < nrows; b += 256) s += partial[4 * (size_t)b + q];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int k = 128; k > 0; k >>= 1) {
+        if (tid < k) red[threadIdx.x] += red[threadIdx.x + k];
+        __syncthreads();
+    }
+    if (tid == 0) out[q] = red[threadIdx.x];
+    if (threadIdx.x != 0) return;
+    const double rr = red[512], ri = red[768];
+    cdiv(rr, ri, st[0], st[1], st[2], st[3]);
+    st[0] = rr;
+    st[1] = ri;
+}
+
+// p = r + beta p, beta = st[2..4)
+__global__ void k_cocg_dir(const double2 *__restrict__ r, double2 *__restrict__ p, const double *__restrict__ st,
+                           size_t nelem)
+{
+    const double br = st[2], bi = st[3];
+    const size_t stride = (size_t)blockDim.x * gridDim.x;
+    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < nelem; e += stride) {
+        const double2 x = r[e], y = p[e];
+        p[e] = make_double2(x.x + br * y.x - bi * y.y, x.y + br * y.y + bi * y.x);
+    }
 }
 
 // y = a_c x + b_c y  (complex scalars per column)
@@ -1045,14 +1094,52 @@ int cocg_update(pned_ctx *ctx, const pned_vec *p, const pned_vec *y, pned_vec *x
     PNED_TRY(ensure_partial(ctx, (size_t)grid * 4));
     if (p->dtype == PNED_C128)
         hipLaunchKernelGGL(k_cocg_update<double>, dim3(grid), dim3(RED_TPB), 0, ctx->stream, (const double2 *)p->data,
-                           (const double2 *)y->data, (double2 *)x->data, (double2 *)r->data, a[0], a[1], nelem,
+                           (const double2 *)y->data, (double2 *)x->data, (double2 *)r->data, a[0], a[1], nullptr,
+                           nullptr, nelem,
                            ctx->d_partial);
     else
         hipLaunchKernelGGL(k_cocg_update<float>, dim3(grid), dim3(RED_TPB), 0, ctx->stream, (const float2 *)p->data,
-                           (const float2 *)y->data, (float2 *)x->data, (float2 *)r->data, a[0], a[1], nelem,
+                           (const float2 *)y->data, (float2 *)x->data, (float2 *)r->data, a[0], a[1], nullptr,
+                           nullptr, nelem,
                            ctx->d_partial);
     PNED_HIP(hipGetLastError());
     return finish_reduce(ctx, grid, 4, out4);
+}
+
+int cocg_start(pned_ctx *ctx, const pned_vec *p, const pned_vec *y, const pned_vec *x, const pned_vec *r,
+               const double *rho, double **st)
+{
+    PNED_TRY(same_shape(p, y));
+    PNED_TRY(same_shape(p, x));
+    PNED_TRY(same_shape(p, r));
+    if (p->nvec != 1 || p->dtype != PNED_C128)
+        return fail(PNED_E_UNSUPPORTED, "cocg steps on the device: one complex128 column");
+    PNED_TRY(ensure_partial(ctx, (size_t)RED_GRID * 4));
+    PNED_TRY(ensure_result(ctx, 4));
+    const double init[4] = {rho[0], rho[1], 0.0, 0.0};
+    return upload_scalars(ctx, init, 4, st);
+}
+
+int cocg_direction(pned_ctx *ctx, const pned_vec *r, pned_vec *p, const double *st)
+{
+    hipLaunchKernelGGL(k_cocg_dir, dim3(grid_for((size_t)p->dim, 256)), dim3(256), 0, ctx->stream,
+                       (const double2 *)r->data, (double2 *)p->data, st, (size_t)p->dim);
+    PNED_HIP(hipGetLastError());
+    return PNED_OK;
+}
+
+int cocg_step(pned_ctx *ctx, const pned_vec *p, const pned_vec *y, pned_vec *x, pned_vec *r, double *st, double *rr)
+{
+    hipLaunchKernelGGL(k_cocg_update<double>, dim3(RED_GRID), dim3(RED_TPB), 0, ctx->stream, (const double2 *)p->data,
+                       (const double2 *)y->data, (double2 *)x->data, (double2 *)r->data, 0.0, 0.0, st, ctx->d_result,
+                       (size_t)p->dim, ctx->d_partial);
+    PNED_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_cocg_end, dim3(1), dim3(1024), 0, ctx->stream, ctx->d_partial, RED_GRID, ctx->d_result, st);
+    PNED_HIP(hipGetLastError());
+    PNED_HIP(hipMemcpyAsync(ctx->h_result, ctx->d_result, sizeof(double) * 4, hipMemcpyDeviceToHost, ctx->stream));
+    PNED_HIP(hipStreamSynchronize(ctx->stream));
+    *rr = ctx->h_result[0];
+    return PNED_OK;
 }
 
 int lanczos_lazy_restore(pned_ctx *ctx, pned_vec *v1, pned_vec *v0, bool swapped, double sx, double a)
