@@ -477,8 +477,9 @@ __global__ __launch_bounds__(TPB) void hv_spin_pass(const double2 *__restrict__ 
 // uniform and a bond whose two sites are both lane digits has one coefficient for the S
 // slots of a thread.  The class loop is bound by LDS reads (16 bytes a lane for each partner),
 // and the rest is one serial chain: address tables, v1, barrier, classes, v0.
-// us per H.v with its read-back, hv_spin_pass -> this: spin 1 on 8 sites 60 -> 30, on 12 sites
-// 140 -> 66; 5 states a site, 8 sites 86 -> 70.
+// us per H.v with its read-back, hv_spin_pass -> this: spin 1 on 8 sites 60 -> 28, on 12 sites
+// 140 -> 62 (3 passes); 4 states a site, 8 sites 51 -> 34; 5 states, 8 sites 86 -> 70.  The same slots
+// on whole large tiles lose: 12 waves hide less than hv_spin_pass's 16 (16 sites 1.95 to 1.83 ms).
 template <int Q, int NR, int TPB, int S, bool CPLX>
 __global__ __launch_bounds__(TPB) void hv_spin_split(const double2 *__restrict__ v1, double2 *__restrict__ v0,
                                                      const SpinPassDev *__restrict__ pd, SpinPassArgs a,
