@@ -268,8 +268,16 @@ struct SpinPassArgs {
     double xs;                        // v0 += xs (H v1); <v1|.> then carries one factor xs
     double ys;                        // first pass: factor on the v0 input
     double zr, zi;                    // first pass: v0 += (zr + i zi) v1 (complex diagonal shift)
+    int nt;                           // 1: v1 streamed non-temporally (4 states a site)
     int dotu;                         // 1: accumulate sum v1 * (H v1) without the conjugate
 };
+
+__device__ __forceinline__ double2 ld_nt2(const double2 *p)
+{
+    using X = double __attribute__((ext_vector_type(2)));
+    const X t = __builtin_nontemporal_load(reinterpret_cast<const X *>(p));
+    return make_double2(t.x, t.y);
+}
 
 // Slots are visited in sweeps of S; a sweep is skipped by the waves that hold no state of the
 // tile in its first slot, and within a sweep every slot is computed (a slot beyond the tile
@@ -347,7 +355,7 @@ __global__ __launch_bounds__(TPB) void hv_spin_pass(const double2 *__restrict__ 
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             if (tid + TPB * r < a.tsz) {
-                const double2 t = v1[base + offj[r]];
+                const double2 t = (Q == 4 && a.nt) ? ld_nt2(&v1[base + offj[r]]) : v1[base + offj[r]];
                 xr[r] = t.x;
                 xi[r] = t.y;
             }
@@ -1203,6 +1211,7 @@ int launch_hv_spin_tiled_shift(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, 
         PNED_HIP(hipMalloc(&ctx->spin_pd, sizeof(SpinPassDev) * np));
         PNED_HIP(hipMemcpy(ctx->spin_pd, plan.dev.data(), sizeof(SpinPassDev) * np, hipMemcpyHostToDevice));
         ctx->spin_K = plan.K;
+        ctx->spin_L = plan.L;
         ctx->spin_np = np;
         ctx->spin_nb.clear();
         for (const auto &b : plan.bonds) ctx->spin_nb.push_back((int)b.size());
@@ -1234,6 +1243,11 @@ int launch_hv_spin_tiled_shift(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, 
         a.zr = zr;
         a.zi = zi;
         a.dotu = dotu ? 1 : 0;
+        // a v1 that fills the 256 MB Infinity Cache alone, where tiles read whole 128-byte lines (4
+        // states a site, two low sites or more: 256-byte runs), leaves the cache to v0 (12 sites 681 ->
+        // 575 us per H.v; v0 non-temporal as well 608, v0 alone 667; runs of 3 and 5 states end in
+        // partial lines, spin 1 on 16 sites 1.99 ms either way)
+        a.nt = q == 4 && ctx->spin_L >= 2 && 16.0 * (double)ctx->dim >= 256.0 * (1 << 20) ? 1 : 0;
         int grid = 0;
         const SpinPassDev *pd = reinterpret_cast<const SpinPassDev *>(ctx->spin_pd) + p;
         double *part = ctx->d_partial + 2 * (size_t)rows;

@@ -257,7 +257,7 @@ struct pned_ctx {
     int num_cu = 0;                  // compute units of the device (read on first use)
     int use_graphs = 1;              // Krylov loops replay captured HIP graphs of their steps
     void *spin_pd = nullptr;         // tiled-pass tables
-    int spin_K = -1, spin_np = 0;
+    int spin_K = -1, spin_L = 0, spin_np = 0;
     std::vector<int> spin_nb, spin_tsz, spin_nlo, spin_ncls, spin_cplx;
     std::vector<int> spin_split;     // per pass: blocks per tile (hv_spin_split), 0 hv_spin_pass, -1 not decided
     // scratch for reductions: per-block partials and final results (pinned host mirror)

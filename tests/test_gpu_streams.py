@@ -57,9 +57,10 @@ def test_split_matches_tiles(spec, cols, dtype):
 
 
 # hv_spin_split against the per-state gather kernel: one tile, several, parts of one and of q
-# slots, complex coefficients (field), tiles of few states, and tiles too many for it (hv_spin_pass)
+# slots, complex coefficients (field), tiles of few states, and tiles too many for it (hv_spin_pass;
+# 4 states on 12 sites with a non-temporal v1)
 @pytest.mark.parametrize("spec,q,tile", [("2x2", 3, 0), ("2x2", 3, 6), ("2x3", 3, 0), ("2x3", 3, 7), ("2x3", 3, 4),
-                                         ("2x2", 4, 0), ("2x2", 4, 4), ("2x2", 5, 0), ("2x2", 5, 3)])
+                                         ("2x2", 4, 0), ("2x2", 4, 4), ("2x3", 4, 0), ("2x2", 5, 0), ("2x2", 5, 3)])
 @pytest.mark.parametrize("field", [0.0, 0.2])
 def test_spin_split_matches_gather(spec, q, tile, field):
     ctx = gpu.Context(model.build_operator(lattice.get_cluster(spec), 20, 108.0, q=q, field=field))
