@@ -993,6 +993,28 @@ bool split_diag_slots(const DiagDev &dh, uint32_t slot_bits, DiagDev &out)
     return true;
 }
 
+// The passes of an untuned plan from K tile bits: one bit more where that saves a whole pass (a pass
+// streams v1 and v0 once).  One operator per column: only tiles that leave the columns' coefficients room
+// in LDS, down to kmin bits (18 sites with 64 operators and off-diagonal exchange: 7 passes of 2^11-state
+// tiles 2.71 ms, 6 of 2^12 on the state-major kernel, which reads the coefficients from memory, 3.58);
+// where not even those do, kmin bits by the same rule, on the state-major kernel.
+static int s12_untuned_passes(S12Plan &pl, int colbits, int dtype, int K, int kmin, int kmax, int L)
+{
+    for (;; --K) {
+        PNED_TRY(s12_make_passes(pl, colbits, K, L));
+        const bool fits = s12_tm_fits(pl, dtype);
+        if (K < kmax) {
+            S12Plan wider = pl;
+            PNED_TRY(s12_make_passes(wider, colbits, K + 1, L));
+            if (wider.passes.size() < pl.passes.size() && (s12_tm_fits(wider, dtype) || (K <= kmin && !fits))) {
+                pl = std::move(wider);
+                return PNED_OK;
+            }
+        }
+        if (fits || K <= kmin) return PNED_OK;
+    }
+}
+
 int ensure_s12_plan(pned_ctx *ctx, int colbits, int dtype)
 {
     if (ctx->plan_colbits == colbits && ctx->plan_dtype == dtype) return PNED_OK;
@@ -1000,8 +1022,7 @@ int ensure_s12_plan(pned_ctx *ctx, int colbits, int dtype)
     // the whole tile sits in LDS (160 KB on gfx950): 2^13 complex128 or 2^14 complex64.
     // Untuned default: complex128 2^11-state tiles up to 2^21 elements (enough tiles to fill
     // the compute units), 2^12 above; complex64 2^12 up to 2^25 elements, 2^13 above (its rounded
-    // sums follow the passes, so the tiles are part of its results); each one bit more where
-    // that saves a pass
+    // sums follow the passes, so the tiles are part of its results); each by s12_untuned_passes
     const int kmax = (dtype == PNED_C128) ? 13 : 14;
     int K = ctx->tune_tile_bits;
     const bool untuned = K <= 0;
@@ -1011,15 +1032,8 @@ int ensure_s12_plan(pned_ctx *ctx, int colbits, int dtype)
     }
     if (K > kmax) K = kmax;
     int L = ctx->tune_low_bits > 0 ? ctx->tune_low_bits : 3;
-    PNED_TRY(s12_make_passes(ctx->s12, colbits, K, L));
-    if (untuned && K < kmax) {
-        // one tile bit more when it saves a whole pass (a pass streams v1 and v0 once)
-        S12Plan wider;
-        wider.n = ctx->s12.n;
-        wider.terms = ctx->s12.terms;
-        PNED_TRY(s12_make_passes(wider, colbits, K + 1, L));
-        if (wider.passes.size() < ctx->s12.passes.size()) PNED_TRY(s12_make_passes(ctx->s12, colbits, K + 1, L));
-    }
+    if (untuned) PNED_TRY(s12_untuned_passes(ctx->s12, colbits, dtype, K, kmax - 2, kmax, L));
+    else PNED_TRY(s12_make_passes(ctx->s12, colbits, K, L));
     S12Plan &pl = ctx->s12;
     const size_t nt = std::max<size_t>(pl.devterms.size(), 1);
     PNED_HIP(hipStreamSynchronize(ctx->stream));

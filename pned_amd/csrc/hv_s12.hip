@@ -995,6 +995,13 @@ static int launch_pass(pned_ctx *ctx, const void *v1, void *v0, const DiagDev *d
     return PNED_OK;
 }
 
+// the instances of dispatch_pass
+static bool has_pass(int TPB, int R)
+{
+    if (TPB == 256 || TPB == 512) return R <= 32 && R > TPB / 512;
+    return R == 1 && (TPB == 128 || TPB == 64 || TPB == 32 || TPB == 16);
+}
+
 template <typename Real>
 static int dispatch_pass(pned_ctx *ctx, int TPB, int R, const void *v1, void *v0,
                          const DiagDev *ddiag, const PassDev *pd, const PassArgs &a, double *partial, int grid)
@@ -1009,12 +1016,25 @@ static int dispatch_pass(pned_ctx *ctx, int TPB, int R, const void *v1, void *v0
 }
 
 // LDS the term-major kernel stages per-column coefficients in (batch contexts)
-static size_t tm_coef_bytes(const PassArgs &a)
+static size_t tm_coef_bytes(int nop, int nterm, bool diag, size_t ngroups)
 {
-    if (a.nop <= 1) return 0;
-    return sizeof(double) * ((size_t)4 * a.nterm * a.nop + (a.diag ? (size_t)2 * (a.ngroups + 1) * a.nop : 0));
+    if (nop <= 1) return 0;
+    return sizeof(double) * ((size_t)4 * nterm * nop + (diag ? (size_t)2 * (ngroups + 1) * nop : 0));
+}
+static size_t tm_coef_bytes(const PassArgs &a) { return tm_coef_bytes(a.nop, a.nterm, a.diag != 0, a.ngroups); }
+// a pass's tile and coefficients
+static size_t tm_lds(const S12Plan &pl, const PassPlan &pp, bool c128)
+{
+    return ((size_t)(c128 ? 16 : 8) << pp.K) + tm_coef_bytes(pl.nop, pp.nterm, pp.diag, pl.diag.size());
 }
 constexpr size_t LDS_LIMIT = 160 * 1024;
+
+bool s12_tm_fits(const S12Plan &pl, int dtype)
+{
+    for (const PassPlan &pp : pl.passes)
+        if (tm_lds(pl, pp, dtype == PNED_C128) > LDS_LIMIT) return false;
+    return true;
+}
 // a batched tile of a single-operator context holds the columns of one 256-byte run (32
 // complex64 or 16 complex128 values per state); more columns run in groups
 constexpr size_t COL_GROUP_BYTES = 256;
@@ -1296,14 +1316,25 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
     const int TPBpref = small ? 8192 : (ctx->tune_threads == 256 || ctx->tune_threads == 512 || ctx->tune_threads == 1024)
                             ? ctx->tune_threads
                             : (ctx->s12_kernel == 1 ? default_threads(ctx, pl, colbits, c128) : 512);
-    std::vector<int> tpb(npass), rr(npass);
+    std::vector<int> tpb(npass), rr(npass), tmk(npass);   // tmk: the pass takes the term-major kernel
     for (int p = 0; p < npass; ++p) {
+        const PassPlan &pp = pl.passes[p];
         int T = TPBpref;
-        while (T > 16 && T > (1 << pl.passes[p].K)) T >>= 1;
+        while (T > 16 && T > (1 << pp.K)) T >>= 1;
+        tmk[p] = ctx->s12_kernel == 1 && !small &&
+                 (c128 ? has_tm<double>(T, (1 << pp.K) / T) : has_tm<float>(T, (1 << pp.K) / T)) &&
+                 tm_lds(pl, pp, c128) <= LDS_LIMIT;
+        // a default thread count is the term-major kernel's; a pass that leaves it (coefficients beyond
+        // the LDS) runs the state-major kernel on 256 threads, 512 for 2^14 states
+        if (ctx->s12_kernel == 1 && !small && !tmk[p] && ctx->tune_threads == 0)
+            T = std::min(T, pp.K > 13 ? 512 : 256);
         tpb[p] = T;
-        rr[p] = (1 << pl.passes[p].K) / T;
+        rr[p] = (1 << pp.K) / T;
         if (rr[p] > PD_HI) return fail(PNED_E_UNSUPPORTED, "tile too large for the thread count");
-        if ((int)pl.passes[p].ob.size() > 22) return fail(PNED_E_UNSUPPORTED, "too many outer bits");
+        if ((int)pp.ob.size() > 22) return fail(PNED_E_UNSUPPORTED, "too many outer bits");
+        // (before the first launch: v0 is not touched by a call that fails)
+        if (!small && !tmk[p] && !has_pass(T, rr[p]))
+            return fail(PNED_E_UNSUPPORTED, "no H.v kernel instance for this tile shape");
     }
     if (noalloc && ctx->pd_threads != TPBpref)
         return fail(PNED_E_ARG, "no H.v plan for this thread count yet: call pned_p_mltply_v3 once after "
@@ -1433,7 +1464,6 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
         const int TPB = tpb[p], R = rr[p];
         const int grid = pass_grid(p);
         const PassDev *pdp = reinterpret_cast<const PassDev *>(ctx->pd_dev) + p;
-        const size_t tile_bytes = esz * (size_t)TPB * R;
         SmallArgs sm{};
         if (small) {
             sm.colbits = colbits;
@@ -1456,8 +1486,7 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
             sm.tbh = from(pp.K - lsplit);
             for (int k = 0; k < a.nouter; ++k) sm.ob |= (uint64_t)expand(pp.ob[k]) << (5 * k);
         }
-        const bool tm = ctx->s12_kernel == 1 && (c128 ? has_tm<double>(TPB, R) : has_tm<float>(TPB, R)) &&
-                        tile_bytes + tm_coef_bytes(a) <= LDS_LIMIT;
+        const bool tm = tmk[p] != 0;
         const DiagDev *dgp = (pp.diag && ctx->d_diag_tm) ? ctx->d_diag_tm : ctx->d_diag;
         if (!noalloc && lz_fused && p == npass - 1 && p > 0 && (tm || small) && c128 && nvec == 1 && pl.nop <= 1) {
             // deferred-normalisation Lanczos step: this pass's <v1|H v1> share first (no v0

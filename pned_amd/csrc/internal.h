@@ -106,6 +106,8 @@ int s12_decompose(int n, int ibond, const int32_t *ipair, const int32_t *btype,
                   const int8_t *pos = nullptr);
 // group terms into tile passes for a given memory layout
 int s12_make_passes(S12Plan &plan, int colbits, int tile_bits, int low_bits);
+// every pass's tile and staged per-column coefficients fit the term-major kernel's LDS
+bool s12_tm_fits(const S12Plan &plan, int dtype);
 
 // Memory layout of a full-space S=1/2 context: the memory index of basis state s is
 // swap(s), which exchanges nswap disjoint pairs of bits (an involution, so the same map

@@ -1,0 +1,37 @@
+"""Which kernels the host code launches, and in which shape, by size (no GPU: see record.py)."""
+import pytest
+
+from tests.record import record  # noqa: F401  (fixture)
+
+LDS = 160 * 1024
+
+
+def test_batch_contexts_have_a_kernel(record):
+    """One operator per column, complex128 and complex64: every size and operator count gets a kernel
+    whose tile and staged coefficients fit the LDS, on wider tiles only while they do."""
+    got = record("""
+out = []
+for l1, l2 in [(1, 4), (2, 3), (1, 7), (2, 4), (1, 9), (2, 5), (1, 11)]:
+    for cols in (2, 8, 16, 32, 64):
+        for field in (0.0, 0.1):
+            ops = [offdiagonal(l1, l2, 20.0 + c, field) for c in range(cols)]
+            for dtype in (gpu.C128, gpu.C64):
+                if 2 * l1 * l2 + cols.bit_length() - 1 > 26:
+                    continue
+                ctx = gpu.Context(ops[0], batch_ops=ops)
+                x, y = ctx.vector(cols, dtype), ctx.vector(cols, dtype)
+                try:
+                    k = launches(lambda: ctx.hv_fresh(x, y))
+                except gpu.PnedError as e:
+                    k = str(e)
+                out.append([2 * l1 * l2, cols, field, dtype, k])
+print(json.dumps(out))
+""")
+    assert len(got) == 2 * 2 * 33
+    failed = [g[:4] + [g[4]] for g in got if isinstance(g[4], str)]
+    assert not failed, failed
+    for *case, k in got:
+        assert k[-1][0] == "reduce_partials"
+        for name, targs, grid, block, lds, limit in k[:-1]:
+            assert name in ("hv_s12_tm", "hv_s12_pass") and targs[0] == block, (case, name)
+            assert lds <= limit <= LDS, (case, name, lds, limit)

@@ -1,0 +1,41 @@
+"""H.v at sizes where the choice of tile, threads or kernel changes, against the oracle."""
+import numpy as np
+import pytest
+
+import oracle
+from pned_amd import gpu, lattice, model
+
+pytestmark = pytest.mark.gpu
+
+
+def _offdiagonal(cl, phi, field):
+    c = model.set_lattice(20, phi)
+    c.I11, c.I12, c.I11p, c.I12p, c.I11pp, c.I12pp = 0.21, 0.13, 0.21, 0.13, 0.21, 0.13
+    H = model.bond_matrices(c, 2, "s12", field=field)
+    mask, parity = model.local_mask(H, 2, "s12")
+    return model.Operator(cl.n, 2, cl.ipair, cl.ibond_type, H, mask, parity, "s12", 0.0)
+
+
+def _columns(ctx, ops, dtype, tol):
+    """One H.v of a batch context (one operator per column), every column against the oracle."""
+    cols = len(ops)
+    x, y = ctx.vector(cols, dtype), ctx.vector(cols, dtype)
+    ctx.set_initial_vec(x, 5)
+    ctx.set_initial_vec(y, 6)
+    X, Y = x.download().astype(complex), y.download().astype(complex)
+    pr = ctx.p_mltply_v3(x, y, 0.03)
+    got = y.download()
+    for c in {0, 1, cols - 1}:
+        xc, want = np.ascontiguousarray(X[:, c]), Y[:, c].copy()
+        ref = oracle.hv(oracle.OracleOp(ops[c]), xc, want, eperbd=0.03)
+        assert np.linalg.norm(got[:, c] - want) <= tol * np.linalg.norm(want), c
+        assert abs(pr[c] - ref) <= tol * np.linalg.norm(xc) * np.linalg.norm(want - Y[:, c]), c
+
+
+# 18 sites: 2^13-state tiles would save a pass, but leave the columns' coefficients no room in LDS.
+# At most 9 terms a bond and 3 a site, one rounding each: 300 * 1.1e-16 (complex64 6e-8 with 3 roundings a term)
+@pytest.mark.parametrize("cols,dtype,tol", [(16, gpu.C128, 1e-13), (64, gpu.C128, 1e-13), (64, gpu.C64, 2e-5)])
+def test_batch_coefficients_beside_the_tile(cols, dtype, tol):
+    cl = lattice.get_cluster("3x3")
+    ops = [_offdiagonal(cl, 20.0 + 3.0 * c, 0.1 + 0.01 * c) for c in range(cols)]
+    _columns(gpu.Context(ops[0], batch_ops=ops), ops, dtype, tol)
