@@ -79,8 +79,9 @@ int pned_ctx_set_matrices(pned_ctx *ctx, const double *xlocal_ham, const int32_t
  * 0 = default */
 int pned_ctx_tune(pned_ctx *ctx, int tile_bits, int low_bits, int threads);
 /* autotuner (no reference counterpart): times one fresh H.v v1 -> v0 for every
- * (tile bits, forced low bits, threads per block) candidate that fits LDS and keeps the
- * fastest for this context; v0 is overwritten.  Outputs may be NULL. */
+ * (tile bits, forced low bits, threads per block) candidate that fits LDS and for the untuned
+ * plan, and keeps the fastest for this context (the untuned plan, the usual winner on short
+ * vectors, is reported as 0, 0, 0); v0 is overwritten.  Outputs may be NULL. */
 int pned_ctx_autotune(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, int reps, int *best_tile_bits,
                       int *best_low_bits, int *best_threads, double *best_ms);
 /* spin-S kernel choice: 1 = tiled passes (default, q = 3..5), 0 = per-state gather */

@@ -1383,7 +1383,10 @@ int pned_ctx_tune(pned_ctx *ctx, int tile_bits, int low_bits, int threads)
 }
 
 // Autotuner: times one fresh H.v v1 -> v0 for each candidate (tile bits, forced low bits,
-// threads per block) that fits LDS, keeps the fastest (v0 is overwritten).
+// threads per block) that fits LDS and for the untuned plan (0, 0, 0), which alone runs short vectors on
+// hv_s12_split (12 sites: 29.8 us per H.v, the best explicit plan 34.6), and keeps the fastest (v0 is
+// overwritten).  Elsewhere the untuned plan is one of the explicit ones: they keep their numbers unless it
+// is more than 2 % faster, which is what two timings of one plan differ by.
 int pned_ctx_autotune(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, int reps, int *best_tile_bits,
                       int *best_low_bits, int *best_threads, double *best_ms)
 {
@@ -1399,24 +1402,29 @@ int pned_ctx_autotune(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, int reps,
     PNED_HIP(hipEventCreate(&e1));
     double best = 1e300;
     int bk = 0, bl = 0, bt = 0;
+    auto time_plan = [&](int K, int L, int T) -> int {
+        ctx->tune_tile_bits = K;
+        ctx->tune_low_bits = L;
+        ctx->tune_threads = T;
+        ctx->plan_colbits = -1;
+        int rc = launch_hv_s12(ctx, v1, v0, 0.0, true, nullptr);   // warm-up, builds the plan
+        if (rc != PNED_OK) return PNED_OK;
+        PNED_HIP(hipEventRecord(e0, ctx->stream));
+        for (int k = 0; k < reps; ++k) PNED_TRY(launch_hv_s12(ctx, v1, v0, 0.0, true, nullptr));
+        PNED_HIP(hipEventRecord(e1, ctx->stream));
+        PNED_HIP(hipEventSynchronize(e1));
+        float ms = 0.f;
+        PNED_HIP(hipEventElapsedTime(&ms, e0, e1));
+        if (ms / reps < (K == 0 ? 0.98 * best : best)) { best = ms / reps; bk = K; bl = L; bt = T; }
+        return PNED_OK;
+    };
     for (int K = kmax - 2; K <= kmax; ++K)
         for (int L = 3; L <= 4; ++L)
             for (int T : {256, 512, 1024}) {
                 if (T == 1024 && ctx->s12_kernel != 1) continue;   // term-major kernel only
-                ctx->tune_tile_bits = K;
-                ctx->tune_low_bits = L;
-                ctx->tune_threads = T;
-                ctx->plan_colbits = -1;
-                int rc = launch_hv_s12(ctx, v1, v0, 0.0, true, nullptr);   // warm-up, builds the plan
-                if (rc != PNED_OK) continue;
-                PNED_HIP(hipEventRecord(e0, ctx->stream));
-                for (int k = 0; k < reps; ++k) PNED_TRY(launch_hv_s12(ctx, v1, v0, 0.0, true, nullptr));
-                PNED_HIP(hipEventRecord(e1, ctx->stream));
-                PNED_HIP(hipEventSynchronize(e1));
-                float ms = 0.f;
-                PNED_HIP(hipEventElapsedTime(&ms, e0, e1));
-                if (ms / reps < best) { best = ms / reps; bk = K; bl = L; bt = T; }
+                PNED_TRY(time_plan(K, L, T));
             }
+    PNED_TRY(time_plan(0, 0, 0));
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     ctx->tune_tile_bits = bk;

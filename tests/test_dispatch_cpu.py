@@ -35,3 +35,18 @@ print(json.dumps(out))
         for name, targs, grid, block, lds, limit in k[:-1]:
             assert name in ("hv_s12_tm", "hv_s12_pass") and targs[0] == block, (case, name)
             assert lds <= limit <= LDS, (case, name, lds, limit)
+
+
+@pytest.mark.parametrize("cost,keeps", [(0.5, True), (5.0, False)])
+def test_autotune_times_the_untuned_plan(record, cost, keeps):
+    """The untuned plan of a short vector is the only one on hv_s12_split: autotuning keeps it (zeros)
+    where it is the fastest and sets an explicit plan where it is not."""
+    tune, names = record(f"""
+rec.record_cost(b"hv_s12_split", ctypes.c_float({cost}))
+ctx = gpu.Context(model.build_operator(T(2, 3), 20, 126.0, field=0.1))
+x, y = ctx.vector(), ctx.vector()
+r = ctx.autotune(x, y, 2)
+print(json.dumps([[r["tile_bits"], r["low_bits"], r["threads"]], [k[0] for k in launches(lambda: ctx.hv_fresh(x, y))]]))
+""")
+    assert (tune == [0, 0, 0]) == keeps
+    assert ("hv_s12_split" in names) == keeps and ("hv_s12_tm" in names) != keeps
