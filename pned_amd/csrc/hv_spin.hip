@@ -1154,11 +1154,12 @@ static int launch_spin_pass(pned_ctx *ctx, int grid_cap, size_t lds, bool cplx, 
 }
 
 // The same pass by hv_spin_split, where R / S blocks to a tile are resident all at once
-// (S = 1 if that fits, else S = q): returns the grid, or 0 to leave it to hv_spin_pass.
-// Decided once per plan and pass (ctx->spin_split).
+// (S = 1 if that fits, else S = q): sets the grid, or leaves it 0 for hv_spin_pass.
+// Decided once per plan and pass (ctx->spin_split); an instance serves passes and contexts of different
+// LDS sizes, so its limit is set at every launch.
 template <int Q, int NR, int TPB>
 static int launch_spin_split(pned_ctx *ctx, int p, bool cplx, const pned_vec *v1, pned_vec *v0,
-                             const SpinPassDev *pd, const SpinPassArgs &a, double *part)
+                             const SpinPassDev *pd, const SpinPassArgs &a, double *part, int &grid)
 {
     constexpr int R = (NR == 2) ? Q * Q : Q;
     using K = void (*)(const double2 *, double2 *, const SpinPassDev *, SpinPassArgs, double *);
@@ -1176,18 +1177,20 @@ static int launch_spin_split(pned_ctx *ctx, int p, bool cplx, const pned_vec *v1
             int per_cu = 0;
             const int np = (k == k1) ? R : R / Q;
             if (!k || parts > 0 || lds > 160 * 1024) continue;
-            (void)hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            PNED_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k, TPB, lds) != hipSuccess)
                 per_cu = 0;
             const uint64_t fit = std::min<uint64_t>((uint64_t)ctx->num_cu * (uint64_t)per_cu, SP_GRID_CAP);
             if (a.tile_count * (uint64_t)np <= fit) parts = np;
         }
     }
-    if (parts == 0) return 0;
-    const int grid = (int)a.tile_count * parts;
-    hipLaunchKernelGGL(parts == R ? k1 : kq, dim3(grid), dim3(TPB), lds, ctx->stream, (const double2 *)v1->data,
+    if (parts == 0) return PNED_OK;
+    const K k = parts == R ? k1 : kq;
+    PNED_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    grid = (int)a.tile_count * parts;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(TPB), lds, ctx->stream, (const double2 *)v1->data,
                        (double2 *)v0->data, pd, a, part);
-    return grid;
+    return PNED_OK;
 }
 
 int launch_hv_spin_tiled(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double eperbd, bool fresh,
@@ -1257,12 +1260,14 @@ int launch_hv_spin_tiled_shift(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, 
         const bool cplx = ctx->spin_cplx[p] != 0;
         const size_t lds = spin_lds_bytes(a.tsz, a.ncls, qq, cplx, tpb);
         // one thread per state of the tile's low digits, K - 2 (spin 1) or K - 1 of them
-        if (q == 3 && a.K == 8) grid = launch_spin_split<3, 2, 768>(ctx, p, cplx, v1, v0, pd, a, part);
-        else if (q == 3 && a.K >= 2) grid = launch_spin_split<3, 2, 256>(ctx, p, cplx, v1, v0, pd, a, part);
-        else if (q == 4 && a.K == 6) grid = launch_spin_split<4, 1, 1024>(ctx, p, cplx, v1, v0, pd, a, part);
-        else if (q == 4 && a.K >= 2) grid = launch_spin_split<4, 1, 256>(ctx, p, cplx, v1, v0, pd, a, part);
-        else if (q == 5 && a.K == 5) grid = launch_spin_split<5, 1, 640>(ctx, p, cplx, v1, v0, pd, a, part);
-        else if (q == 5 && a.K >= 2) grid = launch_spin_split<5, 1, 128>(ctx, p, cplx, v1, v0, pd, a, part);
+        int split = PNED_OK;
+        if (q == 3 && a.K == 8) split = launch_spin_split<3, 2, 768>(ctx, p, cplx, v1, v0, pd, a, part, grid);
+        else if (q == 3 && a.K >= 2) split = launch_spin_split<3, 2, 256>(ctx, p, cplx, v1, v0, pd, a, part, grid);
+        else if (q == 4 && a.K == 6) split = launch_spin_split<4, 1, 1024>(ctx, p, cplx, v1, v0, pd, a, part, grid);
+        else if (q == 4 && a.K >= 2) split = launch_spin_split<4, 1, 256>(ctx, p, cplx, v1, v0, pd, a, part, grid);
+        else if (q == 5 && a.K == 5) split = launch_spin_split<5, 1, 640>(ctx, p, cplx, v1, v0, pd, a, part, grid);
+        else if (q == 5 && a.K >= 2) split = launch_spin_split<5, 1, 128>(ctx, p, cplx, v1, v0, pd, a, part, grid);
+        PNED_TRY(split);
         if (grid == 0) {
 #define PNED_SPIN_CASE(QV, TV, RV)                                                                                   \
         if (q == QV && tpb == TV && R == RV) {                                                                      \

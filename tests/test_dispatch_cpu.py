@@ -50,3 +50,22 @@ print(json.dumps([[r["tile_bits"], r["low_bits"], r["threads"]], [k[0] for k in 
 """)
     assert (tune == [0, 0, 0]) == keeps
     assert ("hv_s12_split" in names) == keeps and ("hv_s12_tm" in names) != keeps
+
+
+def test_launches_set_their_lds_limit(record):
+    """Every launch runs under a limit of its function that covers its own LDS, also when passes and
+    contexts of different LDS sizes share an instance."""
+    got = record("""
+out = []
+ctxs = []
+for q, l1, l2, f in [(3, 2, 3, 0.0), (3, 2, 2, 0.0), (3, 1, 5, 0.2), (3, 2, 3, 0.2), (4, 2, 2, 0.0), (4, 1, 5, 0.1), (5, 2, 2, 0.1)]:
+    ctx = gpu.Context(model.build_operator(T(l1, l2), 20, 108.0, q=q, field=f))
+    ctxs.append((ctx, ctx.vector(), ctx.vector()))
+for _ in range(2):
+    for ctx, x, y in ctxs:
+        out += launches(lambda: ctx.hv_fresh(x, y))
+print(json.dumps(out))
+""")
+    assert len({(k[0], k[4]) for k in got if k[0] == "hv_spin_split"}) > 6
+    short = [k for k in got if k[4] > k[5]]
+    assert not short, short
