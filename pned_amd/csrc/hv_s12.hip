@@ -48,7 +48,6 @@ struct PassArgs {
     const double *lz_prd;
     int nt;                // term-major kernel: NT_V1 / NT_V0 streams
 };
-constexpr int NT_V1 = 1, NT_V0 = 2;
 
 // Per-pass address tables in device memory (read with scalar loads):
 //   lo[t]  memory-index offset of thread t's slot (tile bits 0..LT-1)
@@ -1220,6 +1219,17 @@ static int contiguous_bits(const std::vector<int> &b)
     return n;
 }
 
+// (see hv_s12_tm) whole 128-byte lines in every pass: one pass with runs of 64 bytes reads each line
+// twice (24 sites with 8 complex64 columns and a field, where the first pass alone has longer runs: 4.75 ms
+// per H.v, 3.86 without the hint)
+int s12_nt_streams(const S12Plan &pl, int dtype, size_t vec_bytes)
+{
+    int run = 31;
+    for (const PassPlan &pp : pl.passes) run = std::min(run, contiguous_bits(pp.tb));
+    if (2 * vec_bytes <= CACHE_BYTES || ((size_t)(dtype == PNED_C128 ? 16 : 8) << run) < 128) return 0;
+    return vec_bytes > CACHE_BYTES ? NT_V1 | NT_V0 : NT_V0;
+}
+
 // Threads of the untuned term-major plan, by its tile size (complex128 figures: one column with
 // field, us per H.v).  2^12-state tiles 1024 threads up to 2^21 elements (N=20 57.9, on 512 68), 512
 // above (N=24 533 against 565: two blocks per CU), but 1024 with columns of one operator (N=20 with
@@ -1433,11 +1443,7 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
         PNED_HIP(hipGetLastError());
         return PNED_OK;
     };
-    // the non-temporal streams (see hv_s12_tm): whole 128-byte lines only
-    const size_t vec_bytes = esz * (size_t)ctx->dim * (size_t)nvec;
-    const int lowrun = pl.passes.empty() ? 0 : contiguous_bits(pl.passes[0].tb);
-    int nt = 0;
-    if (2 * vec_bytes > CACHE_BYTES && (esz << lowrun) >= 128) nt = vec_bytes > CACHE_BYTES ? NT_V1 | NT_V0 : NT_V0;
+    const int nt = s12_nt_streams(pl, v1->dtype, esz * (size_t)ctx->dim * (size_t)nvec);
     int total_rows = 0;
     for (int p = 0; p < npass; ++p) {
         const PassPlan &pp = pl.passes[p];

@@ -108,6 +108,9 @@ int s12_decompose(int n, int ibond, const int32_t *ipair, const int32_t *btype,
 int s12_make_passes(S12Plan &plan, int colbits, int tile_bits, int low_bits);
 // every pass's tile and staged per-column coefficients fit the term-major kernel's LDS
 bool s12_tm_fits(const S12Plan &plan, int dtype);
+// the vectors that a plan's passes stream non-temporally (vec_bytes each)
+constexpr int NT_V1 = 1, NT_V0 = 2;
+int s12_nt_streams(const S12Plan &plan, int dtype, size_t vec_bytes);
 
 // Memory layout of a full-space S=1/2 context: the memory index of basis state s is
 // swap(s), which exchanges nswap disjoint pairs of bits (an involution, so the same map

@@ -1,6 +1,12 @@
 """Which kernels the host code launches, and in which shape, by size (no GPU: see record.py)."""
+import os
+import shutil
+import subprocess
+
+import numpy as np
 import pytest
 
+from pned_amd import gpu, lattice, model
 from tests.record import record  # noqa: F401  (fixture)
 
 LDS = 160 * 1024
@@ -69,3 +75,37 @@ print(json.dumps(out))
     assert len({(k[0], k[4]) for k in got if k[0] == "hv_spin_split"}) > 6
     short = [k for k in got if k[4] > k[5]]
     assert not short, short
+
+
+@pytest.fixture(scope="module")
+def nt_streams(tmp_path_factory):
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(gpu.LIB_PATH) or not os.path.exists(hipcc):
+        pytest.skip("needs libpned_gpu.so and hipcc")
+    d = tmp_path_factory.mktemp("nt")
+    libdir = os.path.dirname(gpu.LIB_PATH)
+    subprocess.run([hipcc, "-O1", "-std=c++17", os.path.join(os.path.dirname(__file__), "native", "nt_streams.cpp"), "-o",
+                    str(d / "nt"), "-L" + libdir, "-lpned_gpu", "-Wl,-rpath," + libdir], check=True, capture_output=True)
+
+    def run(op, colbits, tile_bits, dtype):
+        with open(d / "op.bin", "wb") as f:
+            np.array([op.n, op.ibond, colbits, tile_bits, dtype], dtype=np.int32).tofile(f)
+            np.asarray(op.ipair, dtype=np.int32).tofile(f)
+            np.asarray(op.ibond_type, dtype=np.int32).tofile(f)
+            np.ascontiguousarray(op.fortran_xlocal()).view(np.float64).tofile(f)
+            np.asarray(op.fortran_llocal(), dtype=np.int32).tofile(f)
+        return [int(x) for x in subprocess.run([str(d / "nt"), str(d / "op.bin")], check=True, capture_output=True).stdout.split()]
+
+    return run
+
+
+# vectors within the 256 MB cache, one of two beyond it, both beyond it; in complex64 a plan whose first pass
+# alone reads whole lines (24 sites, a field), and one with whole lines throughout
+@pytest.mark.parametrize("l1,l2,field,colbits,tile_bits,dtype,want", [
+    (2, 5, 0.1, 2, 12, 0, 0), (3, 4, 0.1, 0, 12, 0, 2), (3, 4, 0.1, 1, 13, 0, 3), (3, 4, 0.1, 2, 14, 1, 0),
+    (3, 4, 0.1, 1, 13, 1, 0), (3, 4, 0.1, 4, 13, 1, 3), (1, 13, 0.1, 0, 13, 1, 3), (2, 7, 0.0, 0, 13, 1, 0)])
+def test_streams_need_whole_lines_in_every_pass(nt_streams, l1, l2, field, colbits, tile_bits, dtype, want):
+    op = model.build_operator(lattice.torus(l1, l2), 20, 126.0, field=field)
+    run, nt = nt_streams(op, colbits, tile_bits, dtype)
+    assert nt == want
+    assert nt == 0 or (16, 8)[dtype] << run >= 128
