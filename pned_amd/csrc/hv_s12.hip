@@ -1234,7 +1234,8 @@ int s12_nt_streams(const S12Plan &pl, int dtype, size_t vec_bytes)
 // field, us per H.v).  2^12-state tiles 1024 threads up to 2^21 elements (N=20 57.9, on 512 68), 512
 // above (N=24 533 against 565: two blocks per CU), but 1024 with columns of one operator (N=20 with
 // 8 columns 277 against 344); one operator per column 512 above as well (5 batch steps, N=20 with 8
-// columns 2.41 ms against 2.52).  2^11-state tiles 512: 4 slots a thread, 105 VGPRs against 169 on
+// columns 2.41 ms against 2.52) while two of its blocks fit a CU (20 sites with 64 operators, up to 98 KB a
+// block: 5.39 ms per H.v on 512, 4.60 on 1024).  2^11-state tiles 512: 4 slots a thread, 105 VGPRs against 169 on
 // 256 threads (5 batch steps, N=16 with 8 columns 464 us against 528, N=18 with 2 446 against 497;
 // 1024 threads 1000 against 897 at N=18 with 8).  2^13 1024 (N=28 9.08 ms, on 512 13.9).  complex64:
 // 2^12 512 (N=24 383, on 1024 472), 2^13 1024 (N=28 5.8 ms), 2^14 512 (1024 spill; N=24 with 64 columns
@@ -1246,7 +1247,9 @@ static int default_threads(const pned_ctx *ctx, const S12Plan &pl, int colbits, 
     if (K <= 10) return 256;
     if (K == 11) return 512;
     if (!c128) return K == 13 ? 1024 : 512;
-    return K == 12 && big && (colbits == 0 || pl.nop > 1) ? 512 : 1024;
+    bool two = K == 12 && big && (colbits == 0 || pl.nop > 1);
+    for (const PassPlan &pp : pl.passes) two = two && tm_lds(pl, pp, c128) <= LDS_LIMIT / 2;
+    return two ? 512 : 1024;
 }
 
 // the thread count whose register slots order a pass's terms (see build_tm_terms)
@@ -1425,7 +1428,7 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
     auto pass_grid = [&](int p) {
         const uint64_t tc = 1ull << pl.passes[p].ob.size();
         if (small) return (int)tc;   // at most 2^10, times 2^lsplit <= 4 or 16 workgroups
-        const uint64_t fill = (tpb[p] <= 512 && esz << pl.passes[p].K <= LDS_LIMIT / 2) ? 512 : 256;
+        const uint64_t fill = (tpb[p] <= 512 && tm_lds(pl, pl.passes[p], c128) <= LDS_LIMIT / 2) ? 512 : 256;
         const uint64_t want = std::max<uint64_t>(fill, tc / 8);
         return (int)std::min<uint64_t>(std::min<uint64_t>(tc, want), (uint64_t)grid_cap);
     };

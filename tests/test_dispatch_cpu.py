@@ -109,3 +109,25 @@ def test_streams_need_whole_lines_in_every_pass(nt_streams, l1, l2, field, colbi
     run, nt = nt_streams(op, colbits, tile_bits, dtype)
     assert nt == want
     assert nt == 0 or (16, 8)[dtype] << run >= 128
+
+
+def test_batch_threads_by_blocks_per_cu(record):
+    """2^12-state tiles of a batch context: 512 threads while two blocks fit a CU, else 1024."""
+    got = record("""
+out = []
+for l1, l2, cols in [(2, 5, 8), (1, 11, 8), (2, 5, 64), (1, 9, 64)]:
+    ops = [model.build_operator(T(l1, l2), 20, 126.0 + c, field=0.1) for c in range(cols)]
+    ctx = gpu.Context(ops[0], batch_ops=ops)
+    x, y = ctx.vector(cols), ctx.vector(cols)
+    out.append(launches(lambda: ctx.hv_fresh(x, y))[:-1])
+print(json.dumps(out))
+""")
+    tiles = {name for k in got for name, *_ in k}
+    assert tiles == {"hv_s12_tm"}
+    threads = set()
+    for k in got:
+        if k[0][1][0] * k[0][1][1] == 1 << 12:
+            two = all(2 * lds <= LDS for *_, lds, limit in k)
+            assert all(block == (512 if two else 1024) for _, _, _, block, _, _ in k), k
+            threads.add(k[0][3])
+    assert threads == {512, 1024}
