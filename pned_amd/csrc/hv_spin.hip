@@ -923,8 +923,9 @@ struct SpinPlan {
 
 // Builds the passes for tile sites K (at most, fewer when the tables do not fit) and L forced
 // low sites (0: 3 if that costs no pass over 2, else 2; where both vectors fit the 256 MB
-// Infinity Cache and short runs cost little, 1 if that saves a pass over 2, else 2: spin 1 on
-// 12 sites 2 passes for 3, 62 -> 56 us per H.v; on 16 sites, from HBM, 3 for 4 gain nothing).
+// Infinity Cache and short runs cost little, 2 unless 1 or else 3 saves a pass: spin 1 on
+// 12 sites 2 passes with 1 for 3, 62 -> 56 us per H.v, on 14 sites with field 3 with 3 for 4,
+// 489 -> 449; on 16 sites, from HBM, 3 for 4 gain nothing).
 int spin_make_plan(int n, int q, int ibond, const std::vector<int32_t> &sp, const std::vector<int32_t> &btype,
                    const std::vector<double> &xl, const std::vector<int32_t> &ll, int Kmax, int Lreq, SpinPlan &plan)
 {
@@ -951,10 +952,17 @@ int spin_make_plan(int n, int q, int ibond, const std::vector<int32_t> &sp, cons
                 auto npass = [&](const std::vector<std::vector<int>> &c) {
                     return spin_split(spin_balance(c, sp, n, ibond, w), btype, tcls).size();
                 };
-                auto c1 = spin_cover(n, sp, ibond, K, 1);
-                const bool one = !c1.empty() && (c2.empty() || npass(c1) < npass(c2));
-                cov = one ? c1 : c2;
-                L = one ? 1 : std::min(2, K);
+                cov = c2;
+                L = std::min(2, K);
+                for (int l : {1, 3}) {
+                    // (a cover of 3 forced sites has at least as many sets: looked for where the limit
+                    // on a pass's classes has split some)
+                    if (l == 3 && !cov.empty() && npass(cov) == cov.size()) continue;
+                    auto c = l <= K ? spin_cover(n, sp, ibond, K, l) : std::vector<std::vector<int>>{};
+                    if (c.empty() || (!cov.empty() && npass(c) >= npass(cov))) continue;
+                    cov = c;
+                    L = l;
+                }
             } else {
                 auto c3 = (K >= 3) ? spin_cover(n, sp, ibond, K, 3) : std::vector<std::vector<int>>{};
                 if (!c3.empty() && (c2.empty() || c3.size() <= c2.size())) { cov = c3; L = 3; }

@@ -84,3 +84,11 @@ def test_spin1_n18_cover():
     assert all(len(p["sites"]) == 8 for p in plan["passes"])
     assert len(gpu.spin_plan(op, low_sites=2)["passes"]) >= 5
     assert sorted(b for p in plan["passes"] for b in p["bonds"]) == list(range(op.ibond))
+
+
+@pytest.mark.parametrize("l1,l2,q,h", [(1, 7, 3, 0.2), (1, 7, 3, 0.0), (2, 3, 3, 0.2), (1, 5, 4, 0.1), (2, 2, 5, 0.2)])
+def test_default_low_sites_take_no_extra_pass(l1, l2, q, h):
+    """Vectors within the Infinity Cache: the untuned plan has no more passes than 1, 2 or 3 forced low sites."""
+    op = model.build_operator(lattice.torus(l1, l2), 20, 108.0, q=q, field=h)
+    n = [len(gpu.spin_plan(op, low_sites=low)["passes"]) for low in (0, 1, 2, 3)]
+    assert n[0] == min(n)
