@@ -269,13 +269,15 @@ int launch_hv_sector(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double epe
     PNED_TRY(ensure_s12_plan(ctx, 0, PNED_C128));
     const uint64_t dim = (uint64_t)ctx->dim;
     const int ihf = (ctx->n + 1) / 2, ihf0 = ctx->n / 2;
-    // tables in LDS up to 28 sites (98 KB), from L2 above.  1024 threads share one copy from 2^19
-    // states on (N=24: 108 us a call, against 118-122 on 256 threads), on a grid of resident
-    // blocks that stage it once (512; 256-thread blocks in a partial second round took 152)
+    // tables in LDS up to 28 sites (98 KB), from L2 above.  1024 threads share one copy from 21 sites on,
+    // on a grid of resident blocks that stage it once (512; 256 at 27 and 28 sites, where one block fills a
+    // CU's LDS).  us a call at k of 24 sites, 1024 threads and 256: k=12 103 and 135, k=7 35 and 49, k=3 27
+    // and 29; 26 sites, k=6 28 and 42, k=3 26 and 31; 28 sites, k=6 in a second, partial round of blocks 51,
+    // resident 48 (k=14 1635 and 1649); 20 sites, k=10 27 and 27, 16 sites, k=8 25.1 and 24.6.
     const size_t tab = (sizeof(uint32_t) << ihf0) + (sizeof(uint16_t) << ihf);
     const bool lds = ihf <= 14;
-    const int tpb = lds && (ihf == 14 || dim >= (1u << 19)) ? 1024 : 256;
-    const uint64_t cap = tpb == 1024 ? 512 : 4096;
+    const int tpb = lds && ihf >= 11 ? 1024 : 256;
+    const uint64_t cap = tpb == 256 ? 4096 : ihf == 14 ? 256 : 512;
     const int grid = (int)std::min<uint64_t>((dim + tpb - 1) / tpb, cap);
     PNED_TRY(ensure_partial(ctx, 2 * (size_t)grid));
     PNED_TRY(ensure_result(ctx, 8));

@@ -131,3 +131,22 @@ print(json.dumps(out))
             assert all(block == (512 if two else 1024) for _, _, _, block, _, _ in k), k
             threads.add(k[0][3])
     assert threads == {512, 1024}
+
+
+def test_sector_blocks_are_resident(record):
+    """Sector H.v: tables of 12 KB and more in LDS are staged by 1024 threads, on no more blocks than the
+    CUs hold at once."""
+    got = record("""
+out = []
+for l1, l2, k in [(2, 4, 8), (2, 5, 10), (1, 11, 2), (1, 11, 11), (3, 4, 3), (3, 4, 7), (1, 13, 3), (1, 13, 7), (2, 7, 6)]:
+    ctx = gpu.Context(model.build_operator(T(l1, l2), 20, 0.0))
+    ctx.sz_sector(k)
+    x, y = ctx.vector(), ctx.vector()
+    out.append([2 * l1 * l2, launches(lambda: ctx.hv_fresh(x, y))[0]])
+print(json.dumps(out))
+""")
+    for n, (name, targs, grid, block, lds, limit) in got:
+        assert name == "hv_sector_kernel" and targs == [1, n <= 28, block] and lds <= limit
+        assert block == (1024 if 20 < n <= 28 else 256)
+        if block == 1024:   # 16 KB of block sums beside the tables
+            assert grid <= 256 * min(2, LDS // (lds + 16384)), (n, grid, lds)

@@ -39,3 +39,21 @@ def test_batch_coefficients_beside_the_tile(cols, dtype, tol):
     cl = lattice.get_cluster("3x3")
     ops = [_offdiagonal(cl, 20.0 + 3.0 * c, 0.1 + 0.01 * c) for c in range(cols)]
     _columns(gpu.Context(ops[0], batch_ops=ops), ops, dtype, tol)
+
+
+# sectors: 26 sites with few states on 1024 threads, 28 sites with more states than the grid's threads
+@pytest.mark.parametrize("spec,k", [("1x13", 3), ("2x7", 6)])
+def test_sector_grids(spec, k):
+    op = model.build_operator(lattice.get_cluster(spec), 20, 180.0)
+    ctx = gpu.Context(op)
+    ctx.sz_sector(k)
+    x, y = ctx.vector(), ctx.vector()
+    ctx.set_initial_vec(x, 5)
+    ctx.set_initial_vec(y, 6)
+    xh, yh = x.download(), y.download()
+    pr = ctx.p_mltply_v3(x, y, 0.05)
+    want = yh.copy()
+    ref = oracle.hv_sector(oracle.OracleOp(op), k, xh, want, eperbd=0.05)
+    # at most 42 partners a state, each rounded once
+    assert np.linalg.norm(y.download() - want) <= 1e-14 * np.linalg.norm(want)
+    assert abs(pr - ref) <= 1e-13 * np.linalg.norm(xh) * np.linalg.norm(want - yh)
