@@ -150,3 +150,20 @@ print(json.dumps(out))
         assert block == (1024 if 20 < n <= 28 else 256)
         if block == 1024:   # 16 KB of block sums beside the tables
             assert grid <= 256 * min(2, LDS // (lds + 16384)), (n, grid, lds)
+
+
+def test_split_kernel_by_columns(record):
+    """Short vectors: several workgroups per tile up to 2^18 elements in one complex128 column, 2^16 in 2 to
+    16, 2^17 in more and in complex64."""
+    got = record("""
+out = []
+for l1, l2, cols, dtype in [(3, 3, 1, 0), (2, 5, 1, 0), (2, 4, 1, 0), (1, 7, 4, 0), (1, 7, 8, 0), (2, 4, 2, 0), (2, 3, 16, 0), (2, 3, 32, 0), (1, 5, 128, 0),
+                            (1, 7, 8, 1), (2, 4, 2, 1), (2, 4, 4, 1), (3, 3, 1, 1)]:
+    ctx = gpu.Context(model.build_operator(T(l1, l2), 20, 126.0, field=0.1))
+    x, y = ctx.vector(cols, dtype), ctx.vector(cols, dtype)
+    out.append([2 * l1 * l2, cols, dtype, launches(lambda: ctx.hv_fresh(x, y))[0][0]])
+print(json.dumps(out))
+""")
+    for n, cols, dtype, name in got:
+        limit = 17 if dtype == 1 or cols > 16 else 16 if cols > 1 else 18
+        assert (name == "hv_s12_split") == (n + cols.bit_length() - 1 <= limit), (n, cols, dtype, name)
