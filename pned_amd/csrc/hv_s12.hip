@@ -1103,7 +1103,10 @@ static int launch_split(pned_ctx *ctx, const void *v1, void *v0, const TmTerm *t
 }
 
 // log2 of hv_s12_split's workgroups per tile, or -1 where a plan stays with hv_s12_tm: an untuned plan,
-// one operator, tiles of 2^8 .. 2^12 states (2^13 complex64 ones), at most 2^17 elements, or 2^18 in one complex128 column,
+// one operator, tiles of 2^8 .. 2^12 states (2^13 complex64 ones), at most 2^17 elements, or 2^18 in one complex128 column
+// whose passes have 16 terms or more on average (18 sites, two passes: with field, 22 a pass, 68 us per H.v on
+// 256 threads a tile -> 62; without, 13 a pass, 54.9 -> 56.8, and 43 on the 1024 threads it takes now.
+// 1024 threads are faster with field as well, 50 us, but not with the sums of 256 threads bit for bit),
 // or 2^16 in 2 to 16 of them (above, staging a tile several times costs more than the chain: 2^18
 // complex64 elements 49.6 against 47 us per H.v; 2^17 complex128 ones, 512 threads a tile, as 14 sites with
 // 8 columns 36.0 against 32.4, 16 with 2 44.9 against 39.1, but 10 sites with 128 columns, whose tiles hold
@@ -1112,7 +1115,8 @@ static int launch_split(pned_ctx *ctx, const void *v1, void *v0, const TmTerm *t
 static int split_plan(const pned_ctx *ctx, const S12Plan &pl, int colbits, bool c128)
 {
     if (ctx->s12_kernel != 1 || pl.nop > 1 || ctx->tune_threads > 0 || ctx->tune_tile_bits > 0) return -1;
-    if (ctx->n + colbits > (!c128 || colbits > 4 ? 17 : colbits > 0 ? 16 : 18) || pl.passes.empty()) return -1;
+    const bool many = pl.devterms.size() >= 16 * pl.passes.size();
+    if (ctx->n + colbits > (!c128 || colbits > 4 ? 17 : colbits > 0 ? 16 : many ? 18 : 17) || pl.passes.empty()) return -1;
     const int K = pl.passes[0].K;
     for (const PassPlan &pp : pl.passes)
         if (pp.K != K || K < 8 || K > (c128 ? 12 : 13) || pp.ob.size() > 10) return -1;

@@ -167,3 +167,14 @@ print(json.dumps(out))
     for n, cols, dtype, name in got:
         limit = 17 if dtype == 1 or cols > 16 else 16 if cols > 1 else 18
         assert (name == "hv_s12_split") == (n + cols.bit_length() - 1 <= limit), (n, cols, dtype, name)
+
+
+@pytest.mark.parametrize("l1,l2,field,split", [(3, 3, 0.0, False), (3, 3, 0.1, True), (1, 9, 0.0, False), (2, 4, 0.0, True)])
+def test_split_kernel_by_terms(record, l1, l2, field, split):
+    """2^18 elements in one column take the split kernel where the passes have many terms."""
+    names = record(f"""
+ctx = gpu.Context(model.build_operator(T({l1}, {l2}), 20, 126.0, field={field}))
+x, y = ctx.vector(), ctx.vector()
+print(json.dumps([k[0] for k in launches(lambda: ctx.hv_fresh(x, y))]))
+""")
+    assert (names[0] == "hv_s12_split") == split
