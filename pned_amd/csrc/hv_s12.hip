@@ -1115,6 +1115,7 @@ static int launch_split(pned_ctx *ctx, const void *v1, void *v0, const TmTerm *t
 static int split_plan(const pned_ctx *ctx, const S12Plan &pl, int colbits, bool c128)
 {
     if (ctx->s12_kernel != 1 || pl.nop > 1 || ctx->tune_threads > 0 || ctx->tune_tile_bits > 0) return -1;
+    if (colbits > 8) return -1;   // its sums follow those of 256 threads, one column each at most
     const bool many = pl.devterms.size() >= 16 * pl.passes.size();
     if (ctx->n + colbits > (!c128 || colbits > 4 ? 17 : colbits > 0 ? 16 : many ? 18 : 17) || pl.passes.empty()) return -1;
     const int K = pl.passes[0].K;

@@ -178,3 +178,16 @@ x, y = ctx.vector(), ctx.vector()
 print(json.dumps([k[0] for k in launches(lambda: ctx.hv_fresh(x, y))]))
 """)
     assert (names[0] == "hv_s12_split") == split
+
+
+@pytest.mark.parametrize("cols,split", [(256, True), (512, False)])
+def test_split_kernel_columns_fit_its_sums(record, cols, split):
+    """hv_s12_split sums as 256 threads would: more columns than that stay with hv_s12_tm, whose block
+    then has a thread for each."""
+    k = record(f"""
+ctx = gpu.Context(model.build_operator(T(2, 2), 20, 126.0, field=0.1))
+x, y = ctx.vector({cols}), ctx.vector({cols})
+print(json.dumps(launches(lambda: ctx.hv_fresh(x, y))))
+""")
+    assert (k[0][0] == "hv_s12_split") == split
+    assert split or k[0][3] >= cols

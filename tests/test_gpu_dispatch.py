@@ -57,3 +57,21 @@ def test_sector_grids(spec, k):
     # at most 42 partners a state, each rounded once
     assert np.linalg.norm(y.download() - want) <= 1e-14 * np.linalg.norm(want)
     assert abs(pr - ref) <= 1e-13 * np.linalg.norm(xh) * np.linalg.norm(want - yh)
+
+
+# more columns than hv_s12_split can sum (8 sites, 2^17 elements): <x|Hx> of every column
+def test_512_columns():
+    op = model.build_operator(lattice.get_cluster("2x2"), 20, 126.0, field=0.1)
+    ctx = gpu.Context(op)
+    rng = np.random.default_rng(3)
+    xh, yh = (rng.standard_normal((256, 512)) + 1j * rng.standard_normal((256, 512)) for _ in range(2))
+    x, y = ctx.vector(512), ctx.vector(512)
+    x.upload(xh)
+    y.upload(yh)
+    pr = ctx.p_mltply_v3(x, y, 0.03)
+    got = y.download()
+    for c in (0, 1, 255, 256, 300, 511):
+        want = yh[:, c].copy()
+        ref = oracle.hv(oracle.OracleOp(op), np.ascontiguousarray(xh[:, c]), want, eperbd=0.03)
+        assert np.linalg.norm(got[:, c] - want) <= 1e-13 * np.linalg.norm(want), c
+        assert abs(pr[c] - ref) <= 1e-13 * np.linalg.norm(xh[:, c]) * np.linalg.norm(want - yh[:, c]), c
