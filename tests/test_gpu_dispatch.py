@@ -75,3 +75,50 @@ def test_512_columns():
         ref = oracle.hv(oracle.OracleOp(op), np.ascontiguousarray(xh[:, c]), want, eperbd=0.03)
         assert np.linalg.norm(got[:, c] - want) <= 1e-13 * np.linalg.norm(want), c
         assert abs(pr[c] - ref) <= 1e-13 * np.linalg.norm(xh[:, c]) * np.linalg.norm(want - yh[:, c]), c
+
+
+# complex couplings, which the real instances leave out: tables in LDS under 256 and 1024 threads, in memory
+@pytest.mark.parametrize("spec,k", [("2x4", 8), ("1x11", 4), ("1x15", 2)])
+def test_sector_complex_coefficients(spec, k):
+    op = model.build_operator(lattice.get_cluster(spec), 20, 0.0)
+    op.xlocal = op.xlocal * (1.0 + 0.3j)
+    ctx = gpu.Context(op)
+    ctx.sz_sector(k)
+    x, y = ctx.vector(), ctx.vector()
+    ctx.set_initial_vec(x, 5)
+    ctx.set_initial_vec(y, 6)
+    xh, yh = x.download(), y.download()
+    pr = ctx.p_mltply_v3(x, y, 0.05)
+    want = yh.copy()
+    ref = oracle.hv_sector(oracle.OracleOp(op), k, xh, want, eperbd=0.05)
+    # at most 45 partners a state, four products each
+    assert np.linalg.norm(y.download() - want) <= 3e-14 * np.linalg.norm(want)
+    assert abs(pr - ref) <= 1e-13 * np.linalg.norm(xh) * np.linalg.norm(want - yh)
+    assert abs(pr.imag) > 1e-3 * abs(pr)
+
+
+# COCG on the tiled kernel (shift, p^T y and scalars on the device) against the per-state gather kernel and
+# the host's scalars: the same iterates after a few steps, also where the run ends without convergence
+@pytest.mark.parametrize("spec,q", [("2x2", 3), ("2x2", 4), ("2x2", 5)])
+def test_cocg_paths(spec, q):
+    op = model.build_operator(lattice.get_cluster(spec), 20, 108.0, q=q)
+    got = []
+    for tiled in (True, False):
+        ctx = gpu.Context(op)
+        ctx.spin_kernel(tiled)
+        b, x, r, p, y = (ctx.vector() for _ in range(5))
+        ctx.set_initial_vec(b, 9)
+        with pytest.raises(gpu.PnedError) as e:
+            ctx.cocg(-5.0, 1.0, b, x, r, p, y, max_it=4, tol=1e-11)
+        assert e.value.code == gpu.E_NOCONV
+        got.append([v.download() for v in (x, r, p)])
+        it, resid = ctx.cocg(-5.0, 1.0, b, x, r, p, y, tol=1e-11)
+        assert resid < 1e-11
+        # (H - e0 + i eta) x = b
+        xh, bh = x.download(), b.download()
+        ctx.hv_fresh(x, y, -5.0 / op.ibond)
+        assert np.linalg.norm(y.download() + 1j * xh - bh) <= 1e-10 * np.linalg.norm(bh)
+        got[-1].append(xh)
+    # four steps grow a rounding difference of 1e-15 by the condition of the shifted operator, below 100 each
+    for a, c in zip(*got):
+        assert np.linalg.norm(a - c) <= 1e-10 * np.linalg.norm(c)
