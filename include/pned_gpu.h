@@ -87,7 +87,7 @@ int pned_ctx_autotune(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, int reps,
 /* spin-S kernel choice: 1 = tiled passes (default, q = 3..5), 0 = per-state gather */
 int pned_ctx_spin_kernel(pned_ctx *ctx, int tiled);
 /* HIP graph replay in the Krylov loops (no reference counterpart): 1 (default) = pned_lnc1
- * and pned_dsflnc1z on one-column S=1/2 full-space contexts replay their steps between the
+ * and pned_dsflnc1z on one-column S=1/2 contexts (full space, S^z sectors) replay their steps between the
  * host's convergence checks from captured graphs of 5 steps; 0 = every step launched
  * and read back one by one.  Both give the same alpha/beta bit for bit. */
 int pned_ctx_graphs(pned_ctx *ctx, int enable);

@@ -925,7 +925,8 @@ struct SpinPlan {
 // low sites (0: 3 if that costs no pass over 2, else 2; where both vectors fit the 256 MB
 // Infinity Cache and short runs cost little, 2 unless 1 or else 3 saves a pass: spin 1 on
 // 12 sites 2 passes with 1 for 3, 62 -> 56 us per H.v, on 14 sites with field 3 with 3 for 4,
-// 489 -> 449; on 16 sites, from HBM, 3 for 4 gain nothing).
+// 443 -> 408; on 16 sites, from HBM, 3 passes of 3-state runs for 4 of 27-state runs 1.81 ms for 1.87, but
+// in a field, 4 either way, 3.70 for 3.48; 18 sites 4 for 5 the same 19.1 ms).
 int spin_make_plan(int n, int q, int ibond, const std::vector<int32_t> &sp, const std::vector<int32_t> &btype,
                    const std::vector<double> &xl, const std::vector<int32_t> &ll, int Kmax, int Lreq, SpinPlan &plan)
 {
@@ -1255,9 +1256,11 @@ int launch_hv_spin_tiled_shift(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, 
         a.zi = zi;
         a.dotu = dotu ? 1 : 0;
         // a v1 that fills the 256 MB Infinity Cache alone, where tiles read whole 128-byte lines (4
-        // states a site, two low sites or more: 256-byte runs), leaves the cache to v0 (12 sites 681 ->
-        // 575 us per H.v; v0 non-temporal as well 608, v0 alone 667; runs of 3 and 5 states end in
-        // partial lines, spin 1 on 16 sites 1.99 ms either way)
+        // states a site, two low sites or more: 256-byte runs), leaves the cache to v0 (12 sites, 256 MiB a
+        // vector, 714 -> 649 us per H.v; 14 sites, 4 GiB, 10.83 -> 10.59 ms; at 12 sites v0 non-temporal as
+        // well, or v0 alone, gains less; runs of 3 and 5 states end in partial lines, spin 1 on 16 sites
+        // 1.88 -> 1.91 ms, on 18 sites 19.2 -> 20.1).  (The S=1/2 rule, measured on its own passes,
+        // keeps a v1 of just this size cached.)
         a.nt = q == 4 && ctx->spin_L >= 2 && 16.0 * (double)ctx->dim >= 256.0 * (1 << 20) ? 1 : 0;
         int grid = 0;
         const SpinPassDev *pd = reinterpret_cast<const SpinPassDev *>(ctx->spin_pd) + p;
