@@ -1356,10 +1356,10 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
         if (!small && !tmk[p] && !has_pass(T, rr[p]))
             return fail(PNED_E_UNSUPPORTED, "no H.v kernel instance for this tile shape");
     }
-    if (noalloc && ctx->pd_threads != TPBpref)
+    if (noalloc && (ctx->pd_threads != TPBpref || ctx->pd_tpb != tpb))
         return fail(PNED_E_ARG, "no H.v plan for this thread count yet: call pned_p_mltply_v3 once after "
                                 "changing the tuning (that call rebuilds the plan's tables)");
-    if (ctx->pd_threads != TPBpref || ctx->pd_gap != gap || ctx->pd_dev == nullptr) {
+    if (ctx->pd_threads != TPBpref || ctx->pd_tpb != tpb || ctx->pd_gap != gap || ctx->pd_dev == nullptr) {
         std::vector<PassDev> host(npass);
         for (int p = 0; p < npass; ++p) {
             const PassPlan &pp = pl.passes[p];
@@ -1425,6 +1425,7 @@ static int hv_s12_run(pned_ctx *ctx, const pned_vec *v1, pned_vec *v0, double ep
             }
         }
         ctx->pd_threads = TPBpref;
+        ctx->pd_tpb = tpb;
         ctx->pd_gap = gap;
     }
     // blocks per pass: at least 8 contiguous tiles each (so a block's next-tile loads overlap

@@ -254,6 +254,7 @@ struct pned_ctx {
     double *d_colcoef = nullptr;     // batch contexts: per-column term coefficients
     double *d_coldiag = nullptr;     // batch contexts: per-column diagonal weights
     int pd_threads = -1;
+    std::vector<int> pd_tpb;         // threads of each pass that the address tables are for
     int pd_gap = -1;                 // column-group bits the address tables were built for
     int plan_req_colbits = -1;       // column bits of the vectors the current plan was chosen for
     // spin-S

@@ -16,6 +16,7 @@ static std::map<const void *, int> limits;
 static std::string launches;
 static std::map<std::string, float> costs;   // by part of the kernel's name
 static float clock_ms;
+static size_t uploaded;
 static Dim cfg_grid, cfg_block;
 static size_t cfg_lds;
 static void *cfg_stream;
@@ -43,6 +44,8 @@ const char *record_take()
     return out.c_str();
 }
 
+// bytes copied to the device so far
+size_t record_uploaded() { return uploaded; }
 // the time of a launch of a kernel whose name holds `part` (others 1 ms)
 void record_cost(const char *part, float ms) { costs[part] = ms; }
 
@@ -105,8 +108,12 @@ int hipHostMalloc(void **p, size_t n, unsigned) { return alloc(p, n); }
 int hipFree(void *p) { return free(p), 0; }
 int hipFreeAsync(void *p, void *) { return free(p), 0; }
 int hipHostFree(void *p) { return free(p), 0; }
-int hipMemcpy(void *dst, const void *src, size_t n, int) { return copy(dst, src, n); }
-int hipMemcpyAsync(void *dst, const void *src, size_t n, int, void *) { return copy(dst, src, n); }
+int hipMemcpy(void *dst, const void *src, size_t n, int kind)
+{
+    if (kind == 1) uploaded += n;
+    return copy(dst, src, n);
+}
+int hipMemcpyAsync(void *dst, const void *src, size_t n, int kind, void *) { return hipMemcpy(dst, src, n, kind); }
 int hipMemsetAsync(void *, int, size_t, void *) { return 0; }
 int hipStreamCreateWithFlags(void **s, unsigned) { return *s = dummy, 0; }
 int hipStreamDestroy(void *) { return 0; }

@@ -15,6 +15,7 @@ PRELUDE = """
 import ctypes, json, re, sys
 rec = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 rec.record_take.restype = ctypes.c_char_p
+rec.record_uploaded.restype = ctypes.c_size_t
 sys.path.insert(0, sys.argv[2])
 import numpy as np
 from pned_amd import gpu, lattice, model
@@ -42,6 +43,15 @@ def offdiagonal(l1, l2, phi, field):
     H = model.bond_matrices(c, 2, "s12", field=field)
     mask, parity = model.local_mask(H, 2, "s12")
     return model.Operator(cl.n, 2, cl.ipair, cl.ibond_type, H, mask, parity, "s12", 0.0)
+
+def general(n, seed):
+    "all pairs of n sites, random Hermitian bond matrices: every term that two sites can have"
+    rng = np.random.default_rng(seed)
+    pairs = np.array([(a + 1, b + 1) for a in range(n) for b in range(a + 1, n)], dtype=np.int32)
+    H = rng.standard_normal((9, 4, 4)) + 1j * rng.standard_normal((9, 4, 4))
+    H = H + np.conj(np.transpose(H, (0, 2, 1)))
+    return model.Operator(n, 2, pairs.reshape(-1), (np.arange(len(pairs)) % 9 + 1).astype(np.int32), H,
+                          np.zeros(H.shape, dtype=bool), 1, "s12", 0.0)
 """
 
 

@@ -191,3 +191,26 @@ print(json.dumps(launches(lambda: ctx.hv_fresh(x, y))))
 """)
     assert (k[0][0] == "hv_s12_split") == split
     assert split or k[0][3] >= cols
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+def test_coefficients_beyond_the_lds(record, dtype):
+    """64 operators with every two-site term: some passes leave their coefficients no room, so the
+    state-major kernel runs there; the address tables are rebuilt whenever a pass's threads change with the kernel."""
+    first, second, third, bytes1, bytes2 = record(f"""
+ops = [general(8, c) for c in range(64)]
+ctx = gpu.Context(ops[0], batch_ops=ops)
+x, y = ctx.vector(64, {dtype}), ctx.vector(64, {dtype})
+a = launches(lambda: ctx.hv_fresh(x, y))
+ctx.s12_kernel(0)
+n0 = rec.record_uploaded()
+b = launches(lambda: ctx.hv_fresh(x, y))
+n1 = rec.record_uploaded()
+ctx.s12_kernel(1)
+c = launches(lambda: ctx.hv_fresh(x, y))
+print(json.dumps([a, b, c, n1 - n0, rec.record_uploaded() - n1]))
+""")
+    assert first == third
+    assert {(k[0], k[3]) for k in first[:-1]} == {("hv_s12_pass", 256), ("hv_s12_tm", 512 if dtype else 1024)}
+    assert {(k[0], k[3]) for k in second[:-1]} == {("hv_s12_pass", 512)}
+    assert bytes1 > 0 and bytes2 > 0

@@ -122,3 +122,22 @@ def test_cocg_paths(spec, q):
     # four steps grow a rounding difference of 1e-15 by the condition of the shifted operator, below 100 each
     for a, c in zip(*got):
         assert np.linalg.norm(a - c) <= 1e-10 * np.linalg.norm(c)
+
+
+# every two-site term on all pairs of 8 sites, 64 operators: passes beyond the LDS on the state-major kernel,
+# the others term-major, and all of them state-major.  448 products a state, one rounding each: 5e-14 at
+# most (complex64 3e-5)
+@pytest.mark.parametrize("dtype,tol", [(gpu.C128, 1e-13), (gpu.C64, 3e-5)])
+def test_coefficients_beyond_the_lds(dtype, tol):
+    ops = []
+    for c in range(64):
+        rng = np.random.default_rng(c)
+        pairs = np.array([(a + 1, b + 1) for a in range(8) for b in range(a + 1, 8)], dtype=np.int32)
+        H = rng.standard_normal((9, 4, 4)) + 1j * rng.standard_normal((9, 4, 4))
+        H = H + np.conj(np.transpose(H, (0, 2, 1)))
+        ops.append(model.Operator(8, 2, pairs.reshape(-1), (np.arange(28) % 9 + 1).astype(np.int32), H,
+                                  np.zeros(H.shape, dtype=bool), 1, "s12", 0.0))
+    ctx = gpu.Context(ops[0], batch_ops=ops)
+    for kernel in (1, 0, 1):
+        ctx.s12_kernel(kernel)
+        _columns(ctx, ops, dtype, tol)
