@@ -1102,16 +1102,17 @@ static int launch_split(pned_ctx *ctx, const void *v1, void *v0, const TmTerm *t
     return PNED_OK;
 }
 
-// log2 of hv_s12_split's workgroups per tile, or -1 where a plan stays with hv_s12_tm: an untuned plan,
-// one operator, tiles of 2^8 .. 2^12 states (2^13 complex64 ones), at most 2^17 elements, or 2^18 in one complex128 column
-// whose passes have 16 terms or more on average (18 sites, two passes: with field, 22 a pass, 68 us per H.v on
-// 256 threads a tile -> 62; without, 13 a pass, 54.9 -> 56.8, and 43 on the 1024 threads it takes now.
-// 1024 threads are faster with field as well, 50 us, but not with the sums of 256 threads bit for bit),
-// or 2^16 in 2 to 16 of them (above, staging a tile several times costs more than the chain: 2^18
-// complex64 elements 49.6 against 47 us per H.v; 2^17 complex128 ones, 512 threads a tile, as 14 sites with
-// 8 columns 36.0 against 32.4, 16 with 2 44.9 against 39.1, but 10 sites with 128 columns, whose tiles hold
-// few sites and run in many passes, 133 against 141).  Workgroups of 1024 threads where that makes 256 or more of them, else smaller ones,
-// down to 256 threads
+// log2 of hv_s12_split's workgroups per tile, or -1 where a plan stays with hv_s12_tm.  An untuned plan of
+// one operator, tiles of 2^8 .. 2^12 states (2^13 complex64 ones).  Above a number of elements staging a
+// tile several times costs more than the chain (us per H.v, split kernel against whole tiles):
+// - complex64, or more than 16 complex128 columns, 2^17: 2^18 complex64 elements 49.6 against 47; 2^17 as
+//   10 sites with 128 columns, whose tiles hold few sites and run in many passes, 133 against 141
+// - 2 to 16 complex128 columns 2^16: 14 sites with 8 columns 36.0 against 32.4, 16 with 2 44.9 against 39.1
+// - one complex128 column 2^17, or 2^18 where the passes have 16 terms or more on average: 18 sites in two
+//   passes, with field (22 a pass) 62 against 68 on 256 threads, without (13) 56.8 against 54.9, and 43 on
+//   the 1024 threads such a plan takes.  (1024 threads are faster with field as well, 50, but not with the
+//   sums of 256 threads bit for bit.)
+// Workgroups of 1024 threads where that makes 256 or more of them, else smaller ones, down to 256 threads
 static int split_plan(const pned_ctx *ctx, const S12Plan &pl, int colbits, bool c128)
 {
     if (ctx->s12_kernel != 1 || pl.nop > 1 || ctx->tune_threads > 0 || ctx->tune_tile_bits > 0) return -1;
